@@ -98,6 +98,11 @@ hipError_t launch_conv_state_update(const float* p, const float* prev_in, float*
 hipError_t launch_gated_delta(const float* q, const float* k, const float* v, const float* a, const float* b,
                               const float* a_log, const float* dt_bias, const float* state_in, float* state_out,
                               float* o, uint32_t t, uint32_t ldab, bool write_state, hipStream_t s);
+// The recurrence in blocks of 16 tokens (delta_block.hip).
+hipError_t launch_gated_delta_block(const float* q, const float* k, const float* v, const float* a, const float* b,
+                                    const float* a_log, const float* dt_bias, const float* state_in,
+                                    float* state_out, float* o, uint32_t t, uint32_t ldab, bool write_state,
+                                    hipStream_t s);
 // The chunked recurrence (delta_chunk.hip): `ws` holds delta_chunk_ws_floats(t) floats.
 size_t delta_chunk_ws_floats(uint32_t t);
 hipError_t launch_gated_delta_chunked(const float* q, const float* k, const float* v, const float* a, const float* b,

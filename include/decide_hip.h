@@ -70,8 +70,9 @@ extern "C" {
                                 DECIDE_GEMM=baseline, kernels/gemm.rs:56-65) */
 #define DH_DELTA_CHUNKED 2u    /* dh_gated_delta always runs the chunked recurrence */
 #define DH_DELTA_SEQUENTIAL 4u /* dh_gated_delta always runs the token-by-token kernel (with neither flag:
-                                  chunked for t >= DH_DELTA_CHUNK_MIN_T, token by token below; the choice
-                                  decide makes with DECIDE_DELTA, kernels/delta.rs:36-49) */
+                                  chunked for t >= DH_DELTA_CHUNK_MIN_T; below that in blocks of 16 tokens, and
+                                  token by token where one block would do; the choice decide makes with
+                                  DECIDE_DELTA, kernels/delta.rs:36-49) */
 #define DH_DELTA_CHUNK_MIN_T 320u
 
 typedef struct dh_ctx dh_ctx;
@@ -291,8 +292,11 @@ int dh_conv_state_update(dh_ctx* ctx, void* stream, const float* p, const float*
  * states 16-byte aligned. From t = DH_DELTA_CHUNK_MIN_T on (or always, in a
  * context created with DH_DELTA_CHUNKED) the recurrence runs 64 tokens at a
  * time as fp32 matrix products, in a context workspace that dh_warm_up sizes
- * for max_m tokens (a larger t grows it once); below that (or always, with
- * DH_DELTA_SEQUENTIAL) it runs token by token. */
+ * for max_m tokens (a larger t grows it once). Below that it runs in blocks of
+ * 16 tokens in one kernel, without a workspace, and for t <= 16 (or always,
+ * with DH_DELTA_SEQUENTIAL) token by token. The three differ in rounding only;
+ * a token whose inputs are not finite reaches only itself and later tokens
+ * except in its own 64-token chunk of the chunked recurrence. */
 int dh_gated_delta(dh_ctx* ctx, void* stream, const float* q, const float* k, const float* v, const float* a,
                    const float* b, const float* a_log, const float* dt_bias, const float* state_in, float* state_out,
                    float* o, uint32_t t, uint32_t ldab, uint32_t write_state);

@@ -100,6 +100,42 @@ def test_gated_delta_matches_oracle(gpu, kernels_delta_sequential, kernels_delta
     assert orc.rel_frobenius(s1, ws) <= 1e-4, orc.rel_frobenius(s1, ws)
 
 
+@pytest.mark.parametrize("t", [17, 31, 32, 33, 47, 48, 65, 169, 319])
+def test_gated_delta_blocks_match_oracle(gpu, kernels, stream, t):
+    """The 16-token-block kernel (17 <= t < 320 without a flag) at the edges of its blocks and of the pairs of blocks
+    it prepares together, in place, with v only 4-byte aligned. The bound is the fp32 path's: 128-term dot products
+    of a state that 20 blocks update, each rounding about 6e-8 of its value, random in sign."""
+    q, k, v, p, a_log, dt_bias, s0 = _delta_inputs(t, 170)
+    qd, kd, pd, sd = to_dev(q), to_dev(k), to_dev(p), to_dev(s0)
+    vd = to_dev(np.concatenate([np.zeros(1, np.float32), v.ravel()]))
+    o = full((t + 1, NV, DV), np.float32, 7.0)
+    kernels.delta.gated_delta(stream, (qd, 0), (kd, 0), (vd, 4), (pd, LIN_A * 4), (pd, LIN_B * 4), (to_dev(a_log), 0),
+                              (to_dev(dt_bias), 0), (sd, 0), (sd, 0), (o, 0), t, LIN_IN_N, True)
+    sync()
+    wo, ws = orc.gated_delta(q, k, v, p[:, LIN_A:LIN_A + NV], p[:, LIN_B:LIN_B + NV], a_log, dt_bias, s0, t)
+    got = to_host(o)
+    assert (got[t] == 7.0).all(), "a row past T was written"
+    assert orc.rel_frobenius(got[:t], wo) <= 2e-6, orc.rel_frobenius(got[:t], wo)
+    assert orc.rel_frobenius(to_host(sd), ws) <= 2e-6, orc.rel_frobenius(to_host(sd), ws)
+
+
+@pytest.mark.parametrize("what", ["v", "k", "q", "a", "b", "v inf"])
+def test_gated_delta_blocks_keep_a_bad_token_to_itself_and_later_ones(gpu, kernels, kernels_delta_sequential, stream,
+                                                                       what):
+    """One non-finite input at a token inside a block: the outputs and states it reaches are the token-by-token
+    kernel's, no earlier token and no other head."""
+    t, at = 40, 21
+    q, k, v, p, a_log, dt_bias, s0 = _delta_inputs(t, 180)
+    value = np.inf if what == "v inf" else np.nan
+    {"v": v[at, 3], "v inf": v[at, 3], "k": k[at, 2], "q": q[at, 2], "a": p[at, LIN_A:], "b": p[at, LIN_B:]}[what][5] = value
+    got = _run_delta(kernels, stream, q, k, v, p, a_log, dt_bias, s0, t)
+    want = _run_delta(kernels_delta_sequential, stream, q, k, v, p, a_log, dt_bias, s0, t)
+    for x, y in zip(got, want):
+        np.testing.assert_array_equal(np.isfinite(x), np.isfinite(y))
+        assert orc.rel_frobenius(x[np.isfinite(y)], y[np.isfinite(y)]) <= 2e-6
+    assert not np.isfinite(want[0]).all()
+
+
 @pytest.mark.parametrize("impl", ["chunked", "sequential"])
 def test_gated_delta_unit_gate_known_answer(gpu, kernels_delta_sequential, kernels_delta_chunked, stream, impl):
     """decide's known answer (cpu_ref.rs:224-236) through both GPU implementations: one step, beta = 1 (b = 50),
