@@ -32,7 +32,7 @@ constexpr uint32_t kStreamMaxN = 4096;
 
 // Model estimate for one (variant, splits) choice; +inf if the choice is not
 // valid for the shape.
-double plan_estimate_us(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k, uint32_t epi);
+double plan_estimate_us(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k);
 // Builds the plan for (variant, splits), filling the derived fields.
 Plan plan_make(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k, uint32_t epi);
 // The weight-streaming kernel's plan (M <= kStreamMaxM, K % 128 == 0, N % 32 == 0).

@@ -41,7 +41,8 @@ ENGINE_SHAPES = [
     (2560, 6144, Epilogue.StoreF32),  # BASELINE attention group Q|K|V
     (2560, 9216, Epilogue.StoreF32),
 ]
-DEFAULT_MS = [1, 3, 8, 16, 24, 48, 96, 163, 276, 490, 603, 1024, 2307]
+DEFAULT_MS = [1, 3, 8, 12, 16, 20, 24, 28, 32, 40, 48, 56, 64, 80, 96, 112, 128, 144, 163, 176, 200, 230, 256, 276, 320,
+              370, 430, 490, 550, 603, 680, 760, 850, 950, 1024, 1150, 1300, 1500, 1700, 1900, 2100, 2307]
 SPLITS = [1, 2, 3, 4, 6, 8]
 POOL_BYTES = 640 << 20
 
@@ -145,9 +146,10 @@ def main():
     with open(args.out, "w") as f:
         json.dump({"device": "MI355X", "variants": variants(), "results": results,
                    "seconds": round(time.time() - t_start, 1)}, f, indent=1)
-    print("// measured table rows: {k, n, m, variant, splits}", file=sys.stderr)
+    print("// measured table rows: {k, n, m, variant, splits, us}", file=sys.stderr)
     for r in results:
-        print(f"    {{{r['k']}, {r['n']}, {r['m']}, {r['best'][0]}, {r['best'][1]}}},", file=sys.stderr)
+        print(f"    {{{r['k']}, {r['n']}, {r['m']}, {r['best'][0]}, {r['best'][1]}, "
+              f"{r['best'][2]:.1f}f}},", file=sys.stderr)
 
 
 if __name__ == "__main__":

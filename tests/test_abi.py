@@ -166,6 +166,18 @@ def test_planner_invariants_on_random_shapes():
             assert p["order"] == 0, name
 
 
+@pytest.mark.parametrize("kn", [(2560, 12352), (2560, 18432), (4096, 2560), (9216, 2560), (2560, 2048)])
+def test_planner_at_every_row_count(kn):
+    """Every M through the measured range and past its end: the grid covers the output once per split, no split is
+    empty, and no plan pads M by more than one tile."""
+    k, n = kn
+    for m in range(1, 3200):
+        p = plan_for(m, n, k, Epilogue.StoreF32)
+        assert p["workgroups"] == -(-m // p["bm"]) * -(-n // p["bn"]) * p["splits"], (m, p)
+        assert 1 <= p["splits"] <= 8 and p["ws_bytes"] == (p["splits"] * m * n * 4 if p["splits"] > 1 else 0), (m, p)
+        assert p["bm"] <= 2 * max(m, 16), (m, p)
+
+
 def test_tile_order_gives_each_xcd_a_compact_block():
     """The 8 XCDs each take a contiguous run of work ids. At M = 2,307 the down and out projections make
     15 x 16 tiles of 160 x 160 (30 per XCD): in M-fastest order each XCD's run covers all 15 row blocks of X

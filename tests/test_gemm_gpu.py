@@ -427,6 +427,21 @@ def test_config4_projections_m2307(gpu, kernels, stream, kn):
     check_gemm(f"C4 k{k} n{n}", got[rows], want)
 
 
+@pytest.mark.parametrize("m", [29, 41, 72, 136, 215, 350, 720])
+@pytest.mark.parametrize("n,k,epi", [(2048, 2560, Epilogue.StoreF32), (2560, 4096, Epilogue.AddF32),
+                                     (18432, 2560, Epilogue.SwigluF16)])
+def test_rows_between_the_measured_ones(gpu, kernels, stream, m, n, k, epi):
+    """Row counts between the planner's measured ones, where it compares the neighbouring rows' choices at M itself:
+    whatever it picks stores the right values (sampled rows against the oracle)."""
+    x, w = inputs(m, n, k, 90 + m)
+    y0 = synth.normal_f32(synth.seed_for(97), (m, n), 1.0) if epi == Epilogue.AddF32 else None
+    got = run_gemm(kernels, stream, x, w, epi, y0)
+    rows = sample_rows(m, 12, seed=n)
+    y = orc.gemm_nt_f16(x, w, rows=rows)
+    want = swiglu_f16(y) if epi == Epilogue.SwigluF16 else y if y0 is None else y0[rows] + y
+    check_gemm(f"m{m} n{n} k{k} {epi.name}", got[rows], want)
+
+
 # One shape per tile work order the planner picks (dh_gemm_plan.order: 0 = M tiles fastest, g = column stripes
 # in groups of g), each a single planned launch without split-K.
 ORDER_SHAPES = {0: (603, 18432, 2560), 2: (800, 2048, 2560), 3: (2000, 2048, 2560), 4: (1500, 2560, 4096),
