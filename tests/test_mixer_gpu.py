@@ -307,6 +307,22 @@ def test_attention_matches_oracle(gpu, kernels, stream, rows, npos, kind):
     assert e <= 2e-3, f"attention rel. Frobenius {e:.2e}"  # fp16 P operand and fp16 output
 
 
+@pytest.mark.parametrize("rows,first", [(1, 31), (1, 32), (2, 63), (33, 0), (33, 40), (64, 31), (31, 95)])
+def test_attention_at_the_edges_of_tiles_and_halves(gpu, kernels, stream, rows, first):
+    """Positions first .. first + rows - 1: last keys at the ends of a 64-key tile and of its two 32-key halves, whole
+    and partly masked halves, a second query block of one row. Bound: the fp16 weights and output, 2^-11 each, over
+    sums of up to 126 keys (as in test_attention_matches_oracle)."""
+    q, kc, vc, pq, qpos = _attention_case(rows, first + rows, np.arange(first, first + rows), 230)
+    y = full((rows + 1, 4096), np.float16, 7.0)
+    kernels.attn.attention(stream, (to_dev(q), 0), (to_dev(kc), 0), (to_dev(vc), 0), (to_dev(pq), 0), (u32(qpos), 0),
+                           (y, 0), rows, ATT_IN_N)
+    sync()
+    got = to_host(y).astype(np.float32)
+    assert (got[rows] == 7.0).all()
+    want = orc.attention(q.astype(np.float32), qpos, kc.astype(np.float32), vc.astype(np.float32), pq[:, 4096:])
+    assert orc.rel_frobenius(got[:rows], want) <= 2e-3, orc.rel_frobenius(got[:rows], want)
+
+
 def test_attention_key_pieces_keep_rows_independent(gpu, kernels, stream):
     """96 rows at scattered positions: their query blocks' keys are cut into pieces (every 64 keys at the shortest)
     and merged. A row whose position is below 64 sees one piece only and gets bit for bit the result of a call
