@@ -325,12 +325,11 @@ hipError_t launch_gated_rmsnorm_silu(const float* o, const float* z, const float
 
 // ---------------------------------------------------------------------------
 // Zero-centred RMSNorm over a 256-dim head, then RoPE on dims [0, 64) (pairs
-// i, i + 32) at position pos. One wave per head; lane l owns dims 4l .. 4l+3,
+// i, i + 32) at the row's position. One wave per head; lane l owns dims 4l .. 4l+3,
 // so lane l < 8 pairs with lane l + 8 (xor 8). Returns the lane's 4 values.
-__device__ __forceinline__ f4 norm_rope4(f4 x, const float* __restrict__ wn, const float* __restrict__ inv_freq,
-                                         uint32_t pos, int lane) {
+// `cs` and `sn` hold cos and sin of the row's 32 angles, shared by its heads (rope_angles).
+__device__ __forceinline__ f4 norm_rope4(f4 x, const f4& wv, const float* cs, const float* sn, int lane) {
   const float inv = rsqrtf(wave_sum(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3]) / (float)HEAD_DIM + 1e-6f);
-  const f4 wv = *(const f4*)(wn + 4 * lane);
 #pragma unroll
   for (int i = 0; i < 4; ++i) x[i] = x[i] * inv * (1.0f + wv[i]);
   f4 other;
@@ -338,66 +337,81 @@ __device__ __forceinline__ f4 norm_rope4(f4 x, const float* __restrict__ wn, con
   for (int i = 0; i < 4; ++i) other[i] = __shfl_xor(x[i], 8, 64);
   if (lane < 16) {
     const bool lo = lane < 8;
+    const f4 c = *(const f4*)(cs + 4 * (lane & 7)), s = *(const f4*)(sn + 4 * (lane & 7));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = 4 * lane + i;
-      const float ang = (float)pos * inv_freq[d % ROT_HALF];
-      float sn, cs;
-      sincosf(ang, &sn, &cs);
+    for (int i = 0; i < 4; ++i)
       // lo: x = a (dim i), other = b (dim i + 32) → a·c − b·s; hi: x = b, other = a → b·c + a·s
-      x[i] = lo ? x[i] * cs - other[i] * sn : x[i] * cs + other[i] * sn;
-    }
+      x[i] = lo ? x[i] * c[i] - other[i] * s[i] : x[i] * c[i] + other[i] * s[i];
   }
   return x;
 }
 
+// cos and sin of the 32 angles of position pos, once per workgroup: formed by every head, their argument reduction was
+// a third of these kernels' time (2,307 rows: q 14.8 → 10.5 µs, k|v 7.9 → 5.0).
+__device__ __forceinline__ void rope_angles(const float* __restrict__ inv_freq, uint32_t pos, float* cs, float* sn) {
+  if (threadIdx.x < ROT_HALF) {
+    float s, c;
+    sincosf((float)pos * inv_freq[threadIdx.x], &s, &c);
+    cs[threadIdx.x] = c;
+    sn[threadIdx.x] = s;
+  }
+  __syncthreads();
+}
+
 // q heads: rows of pq (stride ldq), head h at column 256 h → qo fp16 [rows][16][256].
-// Grid (4, rows) × 256: four heads per workgroup.
+// Grid rows × 256: a wave takes four heads of the row.
 __global__ __launch_bounds__(256) void q_norm_rope_kernel(const float* __restrict__ pq, const float* __restrict__ qw,
                                                           const float* __restrict__ inv_freq,
                                                           const uint32_t* __restrict__ qpos, _Float16* __restrict__ qo,
                                                           uint32_t ldq) {
+  __shared__ __attribute__((aligned(16))) float cs[ROT_HALF], sn[ROT_HALF];
   const int lane = threadIdx.x & 63;
-  const uint32_t h = blockIdx.x * 4 + (threadIdx.x >> 6), r = blockIdx.y;
-  const f4 x = *(const f4*)(pq + (size_t)r * ldq + h * HEAD_DIM + 4 * lane);
-  const f4 y = norm_rope4(x, qw, inv_freq, qpos[r], lane);
+  const uint32_t h0 = (threadIdx.x >> 6) * 4, r = blockIdx.x;
+  f4 x[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = *(const f4*)(pq + (size_t)r * ldq + (h0 + j) * HEAD_DIM + 4 * lane);
+  const f4 wv = *(const f4*)(qw + 4 * lane);
+  rope_angles(inv_freq, qpos[r], cs, sn);
   typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  *(h4*)(qo + ((size_t)r * 16 + h) * HEAD_DIM + 4 * lane) = h4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const f4 y = norm_rope4(x[j], wv, cs, sn, lane);
+    *(h4*)(qo + ((size_t)r * 16 + h0 + j) * HEAD_DIM + 4 * lane) =
+        h4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]};
+  }
 }
 
 hipError_t launch_q_norm_rope(const float* pq, const float* qw, const float* inv_freq, const uint32_t* qpos,
                               _Float16* qo, uint32_t rows, uint32_t ldq, hipStream_t s) {
   if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(q_norm_rope_kernel, dim3(4, rows), dim3(256), 0, s, pq, qw, inv_freq, qpos, qo, ldq);
+  hipLaunchKernelGGL(q_norm_rope_kernel, dim3(rows), dim3(256), 0, s, pq, qw, inv_freq, qpos, qo, ldq);
   return hipGetLastError();
 }
 
 // k heads (norm + RoPE) into kc and v heads (copied) into vc, fp16 caches
-// [pos][4][256], position pos0 + r. Grid (2, rows) × 256: workgroup x = 0
-// takes the 4 k heads, x = 1 the 4 v heads.
+// [pos][4][256], position pos0 + r. Grid rows × 256: a wave takes a k head and a v head.
 __global__ __launch_bounds__(256) void kv_norm_rope_kernel(const float* __restrict__ pkv, const float* __restrict__ kw,
                                                            const float* __restrict__ inv_freq, _Float16* __restrict__ kc,
                                                            _Float16* __restrict__ vc, uint32_t ldkv, uint32_t kcol,
                                                            uint32_t vcol, uint32_t pos0) {
+  __shared__ __attribute__((aligned(16))) float cs[ROT_HALF], sn[ROT_HALF];
   const int lane = threadIdx.x & 63;
-  const uint32_t jh = threadIdx.x >> 6, r = blockIdx.y, pos = pos0 + r;
-  const float* row = pkv + (size_t)r * ldkv;
+  const uint32_t jh = threadIdx.x >> 6, r = blockIdx.x, pos = pos0 + r;
+  const float* row = pkv + (size_t)r * ldkv + jh * HEAD_DIM + 4 * lane;
   typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  if (blockIdx.x == 1) {
-    const f4 x = *(const f4*)(row + vcol + jh * HEAD_DIM + 4 * lane);
-    *(h4*)(vc + ((size_t)pos * 4 + jh) * HEAD_DIM + 4 * lane) = h4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
-    return;
-  }
-  const f4 x = *(const f4*)(row + kcol + jh * HEAD_DIM + 4 * lane);
-  const f4 y = norm_rope4(x, kw, inv_freq, pos, lane);
-  *(h4*)(kc + ((size_t)pos * 4 + jh) * HEAD_DIM + 4 * lane) = h4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]};
+  const f4 k = *(const f4*)(row + kcol), v = *(const f4*)(row + vcol), wv = *(const f4*)(kw + 4 * lane);
+  rope_angles(inv_freq, pos, cs, sn);
+  const size_t at = ((size_t)pos * 4 + jh) * HEAD_DIM + 4 * lane;
+  *(h4*)(vc + at) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+  const f4 y = norm_rope4(k, wv, cs, sn, lane);
+  *(h4*)(kc + at) = h4{(_Float16)y[0], (_Float16)y[1], (_Float16)y[2], (_Float16)y[3]};
 }
 
 hipError_t launch_kv_norm_rope(const float* pkv, const float* kw, const float* inv_freq, _Float16* kc, _Float16* vc,
                                uint32_t rows, uint32_t ldkv, uint32_t kcol, uint32_t vcol, uint32_t pos0,
                                hipStream_t s) {
   if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(kv_norm_rope_kernel, dim3(2, rows), dim3(256), 0, s, pkv, kw, inv_freq, kc, vc, ldkv, kcol, vcol,
+  hipLaunchKernelGGL(kv_norm_rope_kernel, dim3(rows), dim3(256), 0, s, pkv, kw, inv_freq, kc, vc, ldkv, kcol, vcol,
                      pos0);
   return hipGetLastError();
 }
@@ -428,8 +442,10 @@ __global__ void embed_bf16_kernel(const uint32_t* __restrict__ ids, const uint16
 hipError_t launch_embed_bf16(const uint32_t* ids, const uint16_t* table, float* out, uint32_t t, uint32_t h,
                              hipStream_t s) {
   if (t == 0) return hipSuccess;
-  const uint32_t bx = (h / 8 + 255) / 256;
-  hipLaunchKernelGGL(embed_bf16_kernel, dim3(bx, t), dim3(256), 0, s, ids, table, out, h);
+  // one workgroup per row, as many threads as it has 8-column pieces (2,307 rows of 2,560: 9.7 → 7.3 µs against two
+  // workgroups of 256)
+  const uint32_t threads = std::min<uint32_t>(1024, (h / 8 + 63) / 64 * 64);
+  hipLaunchKernelGGL(embed_bf16_kernel, dim3(1, t), dim3(threads), 0, s, ids, table, out, h);
   return hipGetLastError();
 }
 
