@@ -5,6 +5,8 @@
 // decide counterparts: kernels/head.metal:8-59 (gather_rows_f32/f16,
 // final_head), kernels/rmsnorm.metal:8-30 (rmsnorm_rows). All are HBM- or
 // latency-bound; wave64 shuffles for the reductions.
+#include <algorithm>
+
 #include "dh_kernels.h"
 #include "normal_gen.h"
 
@@ -312,13 +314,20 @@ hipError_t launch_rmsnorm_rows(const float* x, const float* w, _Float16* y, cons
   const bool vec = h % 4 == 0 && h <= 256 * 16 && ld_in % 4 == 0 && ld_out % 4 == 0 && (uintptr_t)x % 16 == 0 &&
                    (uintptr_t)w % 16 == 0 && (uintptr_t)y % 8 == 0;
   if (vec) {
-    if (h <= 256 * 10)
-      hipLaunchKernelGGL(rmsnorm_rows_vec_kernel<10>, dim3(rows), dim3(320), 0, s, x, w, y, rowmap, h, ld_in, ld_out,
-                         add_one ? 1u : 0u, eps);
-    else
-      hipLaunchKernelGGL(rmsnorm_rows_vec_kernel<16>, dim3(rows), dim3(512), 0, s, x, w, y, rowmap, h, ld_in, ld_out,
-                         add_one ? 1u : 0u, eps);
-    return hipGetLastError();
+    // a launch holds fewer than 2^32 threads: more rows than that go in several
+    const uint32_t threads = h <= 256 * 2 ? 64 : h <= 256 * 10 ? 320 : 512, most = UINT32_MAX / threads;
+    const auto kernel = h <= 256 * 2    ? rmsnorm_rows_vec_kernel<2>
+                        : h <= 256 * 10 ? rmsnorm_rows_vec_kernel<10>
+                                        : rmsnorm_rows_vec_kernel<16>;
+    for (uint32_t r0 = 0; r0 < rows;) {
+      const uint32_t n = std::min(most, rows - r0);
+      hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), 0, s, rowmap ? x : x + (size_t)r0 * ld_in, w,
+                         y + (size_t)r0 * ld_out, rowmap ? rowmap + r0 : nullptr, h, ld_in, ld_out, add_one ? 1u : 0u,
+                         eps);
+      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+      r0 += n;
+    }
+    return hipSuccess;
   }
   hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(rows), dim3(256), 0, s, x, w, y, rowmap, h, ld_in, ld_out,
                      add_one ? 1u : 0u, eps);

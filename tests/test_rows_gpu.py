@@ -116,6 +116,38 @@ def test_rmsnorm_rows_matches_oracle(gpu, kernels, stream, add_one):
     assert (to_host(y)[:, h:] == 0).all()
 
 
+@pytest.mark.parametrize("h", [4, 260, 512, 516, 2556, 2560, 2564, 4096])
+def test_rmsnorm_rows_at_the_edges_of_the_row_widths(gpu, kernels, stream, h):
+    """Widths around those where the 16-byte kernel takes another workgroup size. An output is one fp16 rounding
+    (2^-11) of a value whose fp32 sum the oracle adds in another order."""
+    rows = 5
+    x = synth.normal_f32(synth.seed_for(102), (rows, h), 2.0)
+    w = synth.normal_f32(synth.seed_for(103), (h,), 0.3)
+    rowmap = np.array([4, 0, 3, 3, 1], dtype=np.uint32)
+    y = full((rows + 1, h), np.float16, 7.0)
+    kernels.norm.rmsnorm(stream, (to_dev(x), 0), (to_dev(w), 0), (y, 0), (u32(rowmap), 0), rows, h, h, h, True)
+    sync()
+    got = to_host(y).astype(np.float32)
+    assert (got[rows] == 7.0).all()
+    orc.assert_close(f"rmsnorm h{h}", got[:rows], orc.f16_round(orc.rmsnorm(x[rowmap], w, True)), atol=1e-3, rtol=2e-3)
+
+
+def test_rmsnorm_rows_of_more_threads_than_a_launch_holds(gpu, kernels, stream):
+    """A launch holds fewer than 2^32 threads, 64 per row here: rows past that still come out."""
+    rows, h = (2**32 // 64) + 3, 4
+    x = synth.normal_f32(synth.seed_for(104), (8, h), 2.0)
+    w = synth.normal_f32(synth.seed_for(105), (h,), 0.3)
+    rowmap = np.zeros(rows, dtype=np.uint32)
+    rowmap[-6:] = np.arange(1, 7)
+    y = full((rows, h), np.float16, 7.0)
+    kernels.norm.rmsnorm(stream, (to_dev(x), 0), (to_dev(w), 0), (y, 0), (u32(rowmap), 0), rows, h, h, h, True)
+    sync()
+    got = to_host(y)
+    want = orc.f16_round(orc.rmsnorm(x, w, True))
+    orc.assert_close("rmsnorm, last rows", got[-6:].astype(np.float32), want[1:7], atol=1e-3, rtol=2e-3)
+    assert (got[:-6] == got[0]).all()
+
+
 def test_rmsnorm_kat_on_gpu(gpu, kernels, stream):
     """decide's rmsnorm_by_hand (cpu_ref.rs:204-210) on the GPU: [3, 4], w = [1, 1], add_one → 2·x/√12.5."""
     x = np.array([[3.0, 4.0]], dtype=np.float32)
