@@ -7,11 +7,17 @@
 //   S ← γ_15 S + Σ_i (γ_15/γ_i) D_i k_iᵀ,
 // every product an fp32 matrix product on v_mfma_f32_16x16x4_f32. The token
 // by token form of the same recurrence waits about 160 ns per token for its
-// chain of two dot products and two cross-lane sums; here the chain is paid
-// once per 16 tokens. Measured: 169 tokens 31.5 → 21 µs, 319 tokens 56 → 34,
-// 41 tokens 11.0 → 9.4; about 1.35 µs per block, of which the recurrence's own
-// chain is 0.87 (products, one LDS exchange and a barrier, all in sequence)
-// and the rest its share of the matrix cores with the preparation.
+// chain of two dot products and two cross-lane sums; here the chain (products,
+// one LDS exchange and a barrier, all in sequence) is paid once per 16 tokens.
+// Measured: 169 tokens 31.4 → 22.0 µs, 319 tokens 55.5 → 35.3, 41 tokens
+// 10.9 → 10.2; 1.5 µs per block.
+//
+// Accuracy is no less than token by token: no sum runs longer than it must in
+// one accumulator (T·x in four, the update and M·D in two, K Kᵀ and Q Kᵀ in
+// 16), and log g, β and the γ ratios come from fp64. Against 64 bits, over 17
+// to 319 tokens of inputs as the conv forms them: output 0.99e-7 and state
+// 0.73e-7 (token by token 1.05e-7 and 0.84e-7); with one accumulator each, two
+// for K Kᵀ and Q Kᵀ, and fp32 gates 1.60e-7 and 0.93e-7, at 20.7 µs for 169.
 //
 //   * A workgroup is one value head × 16 value rows: 256 workgroups, one per
 //     CU, the 8 of a head (and of the two value heads that share a key head)
@@ -51,7 +57,7 @@ constexpr int NK = 16, DK = 128, NV = 32, DV = 128;
 constexpr int kTok = 16;   // tokens per block
 constexpr int kAhead = 2;  // blocks prepared together, two prep waves each
 constexpr int kLD = 20;    // row stride of a 16 x 16 LDS matrix: conflict-free 4-byte writes and 16-byte reads
-constexpr float kMinLogG = -1e4f;  // exp of it is 0 in fp32; keeps differences of -inf out of the ratios
+constexpr double kMinLogG = -1e4;  // exp of it is 0 in fp32; keeps differences of -inf out of the ratios
 
 struct Prepared {  // what the recurrence and the output need of one block besides q, k, v
   float t[kTok * kLD];
@@ -78,6 +84,11 @@ __device__ __forceinline__ float row_lane(float x) {
 __device__ __forceinline__ f4 mfma4(float a, float b, const f4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+// exp of an fp64 argument to fp32 accuracy: that of its fp32 part, corrected for what the rounding left off.
+__device__ __forceinline__ float exp_of(double x) {
+  const float hi = (float)x, e = expf(hi);
+  return fmaf(e, (float)(x - hi), e);
+}
 __device__ __forceinline__ bool finite(float x) { return __builtin_fabsf(x) < __builtin_inff(); }
 
 constexpr int kRing = 6;             // blocks of q, k and v in LDS
@@ -94,39 +105,48 @@ struct PrepWave {
   int r, g;
   f4 gram;  // K Kᵀ or Q Kᵀ: rows 4g .., column r
 
+  // The 128 terms in kChains sums of their own, added in pairs: in two they were most of the output's error.
   __device__ __forceinline__ void start(const Rows& R) {
-    f4 c0 = f4{0.f, 0.f, 0.f, 0.f}, c1 = c0;
+    constexpr int kChains = 16;
+    f4 c[kChains];
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const int x0 = r * DK + 4 * ((4 * i + g) ^ r), x1 = r * DK + 4 * ((4 * i + 4 + g) ^ r);
-      const f4 k0 = *(const f4*)(R.k + x0), k1 = *(const f4*)(R.k + x1);
-      const f4 l0 = Q ? *(const f4*)(R.q + x0) : k0, l1 = Q ? *(const f4*)(R.q + x1) : k1;
+    for (int i = 0; i < kChains; ++i) c[i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int x = r * DK + 4 * ((4 * i + g) ^ r);
+      const f4 kf = *(const f4*)(R.k + x);
+      const f4 lf = Q ? *(const f4*)(R.q + x) : kf;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        c0 = mfma4(l0[e], k0[e], c0);
-        c1 = mfma4(l1[e], k1[e], c1);
+        f4& to = c[(4 * i + e) % kChains];
+        to = mfma4(lf[e], kf[e], to);
       }
     }
-    gram = c0 + c1;
+#pragma unroll
+    for (int n = kChains / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; ++i) c[i] += c[i + n];
+    gram = c[0];
   }
   // av, bv: the gate inputs of token t0 + r (of the last token past T).
-  __device__ __forceinline__ void gates(float av, float bv, float negA, float bias, uint32_t t0, Prepared& p) {
+  // log g and β in fp64: their fp32 roundings reach every ratio and product of the block.
+  __device__ __forceinline__ void gates(float av, float bv, double negA, double bias, uint32_t t0, Prepared& p) {
     const bool valid = t0 + r < T;
-    const float z = av + bias;
-    float lg = negA * (z > 20.0f ? z : logf(1.0f + expf(z)));
+    const double z = (double)av + bias;
+    double lg = negA * (z > 20.0 ? z : log(1.0 + exp(z)));
     lg = lg < kMinLogG ? kMinLogG : lg;
-    double sum = valid ? (double)lg : 0.0;
+    double sum = valid ? lg : 0.0;
     sum += row_shr<1>(sum);
     sum += row_shr<2>(sum);
     sum += row_shr<4>(sum);
     sum += row_shr<8>(sum);
     if (g == 0) {
       p.sum[r] = sum;
-      p.beta[r] = valid ? 1.0f / (1.0f + expf(-bv)) : 0.0f;
-      p.gam[r] = expf((float)sum);
+      p.beta[r] = valid ? (float)(1.0 / (1.0 + exp(-(double)bv))) : 0.0f;
+      p.gam[r] = exp_of(sum);
     }
     __builtin_amdgcn_wave_barrier();
-    if (g == 0) p.rest[r] = expf((float)(p.sum[kTok - 1] - sum));
+    if (g == 0) p.rest[r] = exp_of(p.sum[kTok - 1] - sum);
   }
   __device__ __forceinline__ void finish(Prepared& p) {
     const double mine = p.sum[r];
@@ -135,7 +155,7 @@ struct PrepWave {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = 4 * g + e;  // row; column r
-      const float ratio = expf((float)(p.sum[i] - mine));
+      const float ratio = exp_of(p.sum[i] - mine);
       if constexpr (Q)
         p.m[i * kLD + r] = i >= r ? ratio * gram[e] : 0.0f;
       else
@@ -221,9 +241,13 @@ __global__ __launch_bounds__(768) void delta_block_kernel(const float* __restric
       const f4 mm = *(const f4*)(p.m + r * kLD + 4 * g), gam = *(const f4*)(p.gam + 4 * g);
       const f4 d = upd[par][lane];
       const uint32_t bad = first_bad[par][lane];
-      f4 ov = gam * ((sq[par][0][lane] + sq[par][1][lane]) + (sq[par][2][lane] + sq[par][3][lane]));
+      f4 o1 = zero, ov = gam * ((sq[par][0][lane] + sq[par][1][lane]) + (sq[par][2][lane] + sq[par][3][lane]));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ov = mfma4(mm[e], d[e], ov);
+      for (int e = 0; e < 4; e += 2) {
+        ov = mfma4(mm[e], d[e], ov);
+        o1 = mfma4(mm[e + 1], d[e + 1], o1);
+      }
+      ov += o1;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const uint32_t tok = c * kTok + 4 * g + e;
@@ -237,7 +261,7 @@ __global__ __launch_bounds__(768) void delta_block_kernel(const float* __restric
   if (wave >= 4) {
     const uint32_t j = (wave >> 1) & 1;
     if (wave & 1) {
-      const float negA = -expf(a_log[h]), bias = dt_bias[h];
+      const double negA = -exp((double)a_log[h]), bias = dt_bias[h];
       PrepWave<true> w{T, r, g, zero};
       float av, bv;
       auto gates_in = [&](uint32_t t0) {
@@ -366,9 +390,8 @@ __global__ __launch_bounds__(768) void delta_block_kernel(const float* __restric
       bad = min(bad, (uint32_t)__shfl_xor((int)bad, 16, 64));
       bad = min(bad, (uint32_t)__shfl_xor((int)bad, 32, 64));
     }
-    f4 d = zero;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) d = mfma4(tt[e], xv[e], d);
+    f4 d = (mfma4(tt[0], xv[0], zero) + mfma4(tt[1], xv[1], zero)) +
+           (mfma4(tt[2], xv[2], zero) + mfma4(tt[3], xv[3], zero));
     sq[par][wave][lane] = q0 + q1;
 #pragma unroll
     for (int t = 0; t < 2; ++t) s[t] *= gend;
@@ -381,11 +404,16 @@ __global__ __launch_bounds__(768) void delta_block_kernel(const float* __restric
           dd[e] = __builtin_nanf("");
         }
     }
+    f4 u[2] = {zero, zero};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < 4; e += 2) {
       s[0] = mfma4(x.kt[0][e], dd[e], s[0]);
       s[1] = mfma4(x.kt[1][e], dd[e], s[1]);
+      u[0] = mfma4(x.kt[0][e + 1], dd[e + 1], u[0]);
+      u[1] = mfma4(x.kt[1][e + 1], dd[e + 1], u[1]);
     }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) s[t] += u[t];
     if (wave == 0) {
       upd[par][lane] = d;
       first_bad[par][lane] = bad;
