@@ -384,6 +384,38 @@ def test_attention_key_pieces_keep_rows_independent(gpu, kernels, stream):
                                        err_msg=f"row {r} at {qpos[r]}")
 
 
+@pytest.mark.parametrize("rows", [1, 96])
+def test_attention_gate_is_divided_exactly(gpu, kernels, stream, rows):
+    """Row 0 sees one key whose values are 1, so its outputs are the gates' σ = 1 / d in fp16, from the attention kernel
+    (1 row) and from the one that merges key pieces (96 rows). The gates give d = 1 + e^-x an exact fp32 value, chosen so
+    that 1 / d rounds to within an ulp of a tie between two fp16 values: one ulp off in the division shows.
+    e < 0.087 keeps the errors of e (three roundings of at most 2^-22 each) below half an ulp of d. Infinite gates
+    give 1, 0 and NaN as they should."""
+    ties = (2 * np.arange(1024) + 1) / 4096 + 0.5
+    d = np.float32(1 / ties[ties > 0.92])[:, None] + np.float32(2.0**-23) * np.arange(-2, 3, dtype=np.float32)
+    d = d[d < np.float32(1.087)]
+    sigma = np.float32(1) / d
+    near = np.abs(sigma.astype(np.float64) * 2048 % 1 - 0.5) <= 2.0**-13  # 2 ulps of 2^-24 in units of 2^-11
+    d, sigma = d[near], sigma[near]
+    assert 200 < len(d) < 4000
+    gate = np.zeros(4096, np.float32)
+    gate[:len(d)] = -np.log(d.astype(np.float64) - 1)
+    gate[-4:] = [np.inf, -np.inf, np.nan, -200.0]
+    want = np.full(4096, 0.5, np.float16)
+    want[:len(d)] = sigma.astype(np.float16)
+    want[-4:] = [1, 0, np.nan, 0]
+    q, kc, vc, pq, qpos = _attention_case(rows, 1001, [0] + [1000] * (rows - 1), 240)
+    vc[0] = 1
+    pq[0, 4096:8192] = gate
+    y = empty((rows, 4096), np.float16)
+    kernels.attn.attention(stream, (to_dev(q), 0), (to_dev(kc), 0), (to_dev(vc), 0), (to_dev(pq), 0), (u32(qpos), 0),
+                           (y, 0), rows, ATT_IN_N)
+    sync()
+    got = to_host(y)[0]
+    print(len(d), "gates,", int((got[:len(d)] != want[:len(d)]).sum()), "differ")
+    np.testing.assert_array_equal(got, want)
+
+
 def test_attention_rows_are_independent_of_their_neighbours(gpu, kernels, stream):
     """Row r's output depends only on its own query, position and cache rows 0..=qpos[r]."""
     rows = 40
