@@ -44,10 +44,11 @@
 //     The 16-byte chunk c of row t sits at chunk c ^ t (values: at c ^ t / 4),
 //     which keeps both the row and the column reads free of bank conflicts.
 //   * Rows past T load row T - 1 and take β = 0, g = 1: they change nothing.
-//   * A non-finite x (x = β(v − γ S k)) may reach only its own token and later
-//     ones, as token by token; the zeros above T's and M's diagonals would
-//     spread it to earlier tokens of the block, so such a block takes its
-//     products from cleaned operands and marks the later tokens afterwards.
+//   * A non-finite x (x = β(v − γ S k)) or D (finite inputs whose products
+//     overflow) may reach only its own token and later ones, as token by
+//     token; the zeros above T's and M's diagonals would spread it to earlier
+//     tokens of the block, so such a block takes its products from cleaned
+//     operands and marks the later tokens afterwards.
 #include "tile_common.h"
 
 namespace dh {
@@ -379,19 +380,29 @@ __global__ __launch_bounds__(768) void delta_block_kernel(const float* __restric
       q1 = mfma4(x.qa[1][e], s[1][e], q1);
     }
     f4 xv = beta * (x.v - gam * ((k0 + k1) + (k2 + k3)));
-    uint32_t bad = kTok;  // the first token of this value row whose x is not finite
-    if (__any(!finite((xv[0] + xv[1]) + (xv[2] + xv[3])))) {
+    // T · x, a sum per step of four tokens
+    auto update = [&] {
+      return (mfma4(tt[0], xv[0], zero) + mfma4(tt[1], xv[1], zero)) +
+             (mfma4(tt[2], xv[2], zero) + mfma4(tt[3], xv[3], zero));
+    };
+    f4 d = update();
+    uint32_t bad = kTok;  // this value row's first token whose x or D is not finite
+    if (__any(!finite((d[0] + d[1]) + (d[2] + d[3])))) {
+      auto first_not_finite = [&](const f4& y) {
+        uint32_t n = kTok;
 #pragma unroll
-      for (int e = 3; e >= 0; --e)
-        if (!finite(xv[e])) {
-          bad = 4 * g + e;
-          xv[e] = 0.0f;
-        }
-      bad = min(bad, (uint32_t)__shfl_xor((int)bad, 16, 64));
-      bad = min(bad, (uint32_t)__shfl_xor((int)bad, 32, 64));
+        for (int e = 3; e >= 0; --e)
+          if (!finite(y[e])) n = 4 * g + e;
+        n = min(n, (uint32_t)__shfl_xor((int)n, 16, 64));
+        return min(n, (uint32_t)__shfl_xor((int)n, 32, 64));
+      };
+      bad = first_not_finite(xv);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!finite(xv[e])) xv[e] = 0.0f;
+      d = update();
+      bad = min(bad, first_not_finite(d));
     }
-    f4 d = (mfma4(tt[0], xv[0], zero) + mfma4(tt[1], xv[1], zero)) +
-           (mfma4(tt[2], xv[2], zero) + mfma4(tt[3], xv[3], zero));
     sq[par][wave][lane] = q0 + q1;
 #pragma unroll
     for (int t = 0; t < 2; ++t) s[t] *= gend;

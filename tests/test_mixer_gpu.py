@@ -151,15 +151,19 @@ def test_gated_delta_blocks_are_as_exact_as_token_by_token(gpu, kernels, kernels
     assert (np.sqrt(err[0]) <= 1.1 * np.sqrt(err[1])).all(), np.sqrt(err / 2)
 
 
-@pytest.mark.parametrize("what", ["v", "k", "q", "a", "b", "v inf"])
+@pytest.mark.parametrize("what", ["v", "k", "q", "a", "b", "v inf", "k overflow"])
 def test_gated_delta_blocks_keep_a_bad_token_to_itself_and_later_ones(gpu, kernels, kernels_delta_sequential, stream,
                                                                        what):
-    """One non-finite input at a token inside a block: the outputs and states it reaches are the token-by-token
-    kernel's, no earlier token and no other head."""
+    """One non-finite input at a token inside a block, or one finite key so large that the products with it overflow:
+    the outputs and states it reaches are the token-by-token kernel's, no earlier token and no other head."""
     t, at = 40, 21
     q, k, v, p, a_log, dt_bias, s0 = _delta_inputs(t, 180)
-    value = np.inf if what == "v inf" else np.nan
-    {"v": v[at, 3], "v inf": v[at, 3], "k": k[at, 2], "q": q[at, 2], "a": p[at, LIN_A:], "b": p[at, LIN_B:]}[what][5] = value
+    if what == "k overflow":
+        k[at, 2] = 1e25  # k·δ reaches 1e49 at this token, and the state with it
+    else:
+        value = np.inf if what == "v inf" else np.nan
+        {"v": v[at, 3], "v inf": v[at, 3], "k": k[at, 2], "q": q[at, 2], "a": p[at, LIN_A:],
+         "b": p[at, LIN_B:]}[what][5] = value
     got = _run_delta(kernels, stream, q, k, v, p, a_log, dt_bias, s0, t)
     want = _run_delta(kernels_delta_sequential, stream, q, k, v, p, a_log, dt_bias, s0, t)
     for x, y in zip(got, want):
