@@ -71,8 +71,8 @@ extern "C" {
 #define DH_DELTA_CHUNKED 2u    /* dh_gated_delta always runs the chunked recurrence */
 #define DH_DELTA_SEQUENTIAL 4u /* dh_gated_delta always runs the token-by-token kernel (with neither flag:
                                   chunked for t >= DH_DELTA_CHUNK_MIN_T; below that in blocks of 16 tokens, and
-                                  token by token where one block would do; the choice decide makes with
-                                  DECIDE_DELTA, kernels/delta.rs:36-49) */
+                                  token by token for t <= 36; the choice decide makes with DECIDE_DELTA,
+                                  kernels/delta.rs:36-49) */
 #define DH_DELTA_CHUNK_MIN_T 320u
 
 typedef struct dh_ctx dh_ctx;
@@ -293,7 +293,7 @@ int dh_conv_state_update(dh_ctx* ctx, void* stream, const float* p, const float*
  * context created with DH_DELTA_CHUNKED) the recurrence runs 64 tokens at a
  * time as fp32 matrix products, in a context workspace that dh_warm_up sizes
  * for max_m tokens (a larger t grows it once). Below that it runs in blocks of
- * 16 tokens in one kernel, without a workspace, and for t <= 16 (or always,
+ * 16 tokens in one kernel, without a workspace, and for t <= 36 (or always,
  * with DH_DELTA_SEQUENTIAL) token by token. The three differ in rounding only;
  * a token whose inputs are not finite reaches only itself and later tokens
  * except in its own 64-token chunk of the chunked recurrence. */

@@ -100,10 +100,10 @@ def test_gated_delta_matches_oracle(gpu, kernels_delta_sequential, kernels_delta
     assert orc.rel_frobenius(s1, ws) <= 1e-4, orc.rel_frobenius(s1, ws)
 
 
-@pytest.mark.parametrize("t", [17, 31, 32, 33, 47, 48, 65, 169, 319])
+@pytest.mark.parametrize("t", [17, 31, 32, 33, 36, 37, 47, 48, 49, 64, 65, 169, 319])
 def test_gated_delta_blocks_match_oracle(gpu, kernels, stream, t):
-    """The 16-token-block kernel (17 <= t < 320 without a flag) at the edges of its blocks and of the pairs of blocks
-    it prepares together, in place, with v only 4-byte aligned. The bound is the fp32 path's: 128-term dot products
+    """The 16-token-block kernel (37 <= t < 320 without a flag) at the edges of its blocks and of the pairs of blocks
+    it prepares together, and the token-by-token kernel just below, in place, with v only 4-byte aligned. The bound is the fp32 path's: 128-term dot products
     of a state that 20 blocks update, each rounding about 6e-8 of its value, random in sign."""
     q, k, v, p, a_log, dt_bias, s0 = _delta_inputs(t, 170)
     qd, kd, pd, sd = to_dev(q), to_dev(k), to_dev(p), to_dev(s0)
@@ -117,6 +117,15 @@ def test_gated_delta_blocks_match_oracle(gpu, kernels, stream, t):
     assert (got[t] == 7.0).all(), "a row past T was written"
     assert orc.rel_frobenius(got[:t], wo) <= 2e-6, orc.rel_frobenius(got[:t], wo)
     assert orc.rel_frobenius(to_host(sd), ws) <= 2e-6, orc.rel_frobenius(to_host(sd), ws)
+
+
+@pytest.mark.parametrize("t", [16, 17, 24, 36])
+def test_gated_delta_short_calls_run_token_by_token(gpu, kernels, kernels_delta_sequential, stream, t):
+    """Up to 36 tokens, where the block kernel would be slower, a context without a flag gives the token-by-token
+    kernel's bits."""
+    inputs = _delta_inputs(t, 160)
+    for x, y in zip(*(_run_delta(ks, stream, *inputs, t) for ks in (kernels, kernels_delta_sequential))):
+        np.testing.assert_array_equal(x.view(np.uint32), y.view(np.uint32))
 
 
 def _delta_exact(q, k, v, p, a_log, dt_bias, s0, t):
