@@ -58,11 +58,7 @@ struct Measured {
 // partials costs what it does there. Choices within 2 % of the fastest count
 // as ties and go to the one that covers the least padded area: sustained, the
 // chip is power-limited, and MFMA work on padding rows costs energy that a
-// burst of launches does not show. Three rows keep a choice 4-7 % behind the
-// best: K|V at 800 and 2000, whose tiles run in work orders no other row has,
-// so that every order stays in use and checked, and down at 1150, whose split
-// needs a larger workspace than 603 rows do (graphs are checked across such a
-// growth).
+// burst of launches does not show.
 const Measured kMeasured[] = {
     {2560, 12352, 1, 22, 1, 16.5f}, {2560, 12352, 3, 22, 1, 16.8f}, {2560, 12352, 8, 0, 4, 17.5f},
     {2560, 12352, 12, 22, 1, 17.3f}, {2560, 12352, 16, 0, 4, 18.4f}, {2560, 12352, 20, 22, 1, 18.3f},
@@ -131,7 +127,7 @@ const Measured kMeasured[] = {
     {9216, 2560, 320, 10, 4, 31.9f}, {9216, 2560, 370, 21, 3, 33.7f}, {9216, 2560, 430, 21, 3, 36.9f},
     {9216, 2560, 490, 4, 6, 40.0f}, {9216, 2560, 550, 14, 4, 41.1f}, {9216, 2560, 603, 14, 4, 42.2f},
     {9216, 2560, 680, 10, 2, 48.3f}, {9216, 2560, 760, 4, 4, 49.5f}, {9216, 2560, 850, 8, 3, 56.9f},
-    {9216, 2560, 950, 5, 4, 60.5f}, {9216, 2560, 1024, 4, 3, 61.3f}, {9216, 2560, 1150, 5, 3, 69.3f},
+    {9216, 2560, 950, 5, 4, 60.5f}, {9216, 2560, 1024, 4, 3, 61.3f}, {9216, 2560, 1150, 14, 2, 65.0f},
     {9216, 2560, 1300, 8, 2, 77.5f}, {9216, 2560, 1500, 4, 2, 82.7f}, {9216, 2560, 1700, 5, 2, 91.7f},
     {9216, 2560, 1900, 5, 2, 97.4f}, {9216, 2560, 2100, 9, 2, 107.7f}, {9216, 2560, 2307, 14, 1, 115.3f},
     {2560, 2048, 1, 22, 3, 8.0f}, {2560, 2048, 3, 22, 4, 8.1f}, {2560, 2048, 8, 22, 4, 8.2f},
@@ -144,10 +140,10 @@ const Measured kMeasured[] = {
     {2560, 2048, 230, 18, 2, 13.0f}, {2560, 2048, 256, 18, 1, 14.0f}, {2560, 2048, 276, 18, 1, 13.4f},
     {2560, 2048, 320, 18, 2, 14.3f}, {2560, 2048, 370, 18, 1, 15.8f}, {2560, 2048, 430, 18, 1, 15.7f},
     {2560, 2048, 490, 18, 1, 16.0f}, {2560, 2048, 550, 18, 1, 16.2f}, {2560, 2048, 603, 20, 1, 17.8f},
-    {2560, 2048, 680, 20, 1, 18.0f}, {2560, 2048, 760, 20, 1, 19.8f}, {2560, 2048, 800, 1, 1, 21.7f},
+    {2560, 2048, 680, 20, 1, 18.0f}, {2560, 2048, 760, 20, 1, 19.8f},
     {2560, 2048, 850, 20, 1, 20.0f}, {2560, 2048, 950, 20, 1, 20.4f}, {2560, 2048, 1024, 15, 1, 21.0f},
     {2560, 2048, 1150, 21, 1, 23.1f}, {2560, 2048, 1300, 15, 1, 22.8f}, {2560, 2048, 1500, 21, 1, 24.8f},
-    {2560, 2048, 1700, 21, 1, 27.2f}, {2560, 2048, 1900, 4, 2, 35.2f}, {2560, 2048, 2000, 2, 1, 36.4f},
+    {2560, 2048, 1700, 21, 1, 27.2f}, {2560, 2048, 1900, 4, 2, 35.2f},
     {2560, 2048, 2100, 14, 1, 33.5f}, {2560, 2048, 2307, 14, 1, 34.9f},
     {2560, 8192, 1, 22, 2, 12.5f}, {2560, 8192, 3, 22, 2, 12.6f}, {2560, 8192, 8, 22, 2, 12.8f},
     {2560, 8192, 12, 22, 2, 13.2f}, {2560, 8192, 16, 22, 2, 13.3f}, {2560, 8192, 20, 22, 2, 13.9f},

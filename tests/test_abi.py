@@ -178,6 +178,14 @@ def test_planner_at_every_row_count(kn):
         assert p["bm"] <= 2 * max(m, 16), (m, p)
 
 
+@pytest.mark.parametrize("m", [800, 2000])
+def test_planner_has_no_row_count_of_its_own(m):
+    """K|V at these row counts: one tile is the fastest over the whole range around them, and the plan is their
+    neighbours' (a choice of their own took 29.6 against 20.0 us at 800 rows)."""
+    plans = [plan_for(v, 2048, 2560, Epilogue.StoreF32) for v in (m - 10, m, m + 10)]
+    assert len({(p["variant"], p["splits"]) for p in plans}) == 1, plans
+
+
 def test_tile_order_gives_each_xcd_a_compact_block():
     """The 8 XCDs each take a contiguous run of work ids. At M = 2,307 the down and out projections make
     15 x 16 tiles of 160 x 160 (30 per XCD): in M-fastest order each XCD's run covers all 15 row blocks of X

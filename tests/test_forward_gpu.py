@@ -160,14 +160,14 @@ def test_forward_delta_implementations_agree(gpu, kernels, kernels_delta_sequent
 
 def test_graph_survives_workspace_growth(gpu):
     """A graph keeps the raw workspace pointers it was captured with. Capture at T = 603 (split-K down and out
-    projections), then run an eager forward at T = 1146 on a fresh context without warm-up, which grows the split-K
+    projections), then run an eager forward at T = 1024 on a fresh context without warm-up, which grows the split-K
     workspace: the replayed graph must still reproduce the eager T = 603 forward (the replaced workspace stays
     allocated until the context is destroyed)."""
     from decide_amd.hip import Stream
     from decide_amd.kernels import Kernels
 
     k = Kernels()
-    cfg = ModelConfig(layers=4, vocab=600, max_tokens=1146, max_answers=3, max_cand=5)
+    cfg = ModelConfig(layers=4, vocab=600, max_tokens=1024, max_answers=3, max_cand=5)
     model = Model(k.ctx, cfg)
     st = Stream()
     s = st.handle
@@ -178,10 +178,10 @@ def test_graph_survives_workspace_growth(gpu):
     graph = model.capture(s, (dev[0], 0), 603, (dev[1], 0), 3, (dev[2], 0), (dev[3], 0), (logits, 0))
     st.synchronize()
     eager = to_host(logits)
-    before = k.gemm.plan(1146, 2560, 9216, 2)["ws_bytes"]
-    long_ids, long_ans, long_cand, long_ncand = _request(1146, cfg.vocab, 3, cfg.max_cand, 451)
+    before = k.gemm.plan(1024, 2560, 9216, 2)["ws_bytes"]
+    long_ids, long_ans, long_cand, long_ncand = _request(1024, cfg.vocab, 3, cfg.max_cand, 451)
     _run(model, k, long_ids, long_ans, long_cand, long_ncand, cfg.max_cand, True)
-    assert before > k.gemm.plan(603, 2560, 9216, 2)["ws_bytes"], "the T = 1146 forward must need a larger workspace"
+    assert before > k.gemm.plan(603, 2560, 9216, 2)["ws_bytes"], "the T = 1024 forward must need a larger workspace"
     for i in range(2):
         logits.copy_from(np.full((3, cfg.max_cand), np.nan, np.float32))
         graph.launch(s)

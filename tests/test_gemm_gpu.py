@@ -444,7 +444,7 @@ def test_rows_between_the_measured_ones(gpu, kernels, stream, m, n, k, epi):
 
 # One shape per tile work order the planner picks (dh_gemm_plan.order: 0 = M tiles fastest, g = column stripes
 # in groups of g), each a single planned launch without split-K.
-ORDER_SHAPES = {0: (603, 18432, 2560), 2: (800, 2048, 2560), 3: (2000, 2048, 2560), 4: (1500, 2560, 4096),
+ORDER_SHAPES = {0: (603, 18432, 2560), 2: (1600, 2560, 1024), 3: (2000, 3072, 1024), 4: (1500, 2560, 4096),
                 6: (2307, 2560, 4096), 8: (1024, 3072, 1024)}
 
 
