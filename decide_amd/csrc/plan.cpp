@@ -1,13 +1,18 @@
 // See plan.h. Two parts:
-//   * a table measured on an MI355X: for decide's engine shapes (K, N) at 40
+//   * a table measured on an MI355X: for decide's engine shapes (K, N) at 42
 //     row counts from 1 to 2307, at most 27 % apart above 16, the fastest
 //     (tile variant, split-K) and its time with weights streaming from HBM —
 //     the MI355X counterpart of decide's M1 Pro RECOMMENDED table
 //     (crates/decide-metal/src/gemm_configs.rs:247-283). `python -m
-//     decide_amd.tune_gemm` times the menu at these rows;
-//   * a cost model for every other shape, fitted to the seven fastest choices
-//     of every table point (rms error 9 %; its pick is 7 % slower than the
-//     fastest on average over those points): a 64-wide K stage takes the
+//     decide_amd.tune_gemm` times the menu at these rows, as the calls the
+//     table's times are of; in a later run of it over all 378 points the
+//     table's choices were 1.2 % from that run's fastest;
+//   * a cost model for every other shape, fitted to the table's points (over
+//     the seven fastest choices of each in that later run: rms error 10 %, its
+//     pick 3.5 % from the fastest). Off the fit, 77 points of seven other
+//     shapes from 3 to 2,200 rows: its pick 9 % from the fastest, mostly below
+//     100 rows; engine shapes at 3,000, 4,096 and 8,192 rows: the fastest, or
+//     within 2 %. A 64-wide K stage takes the
 //     longer of its MFMAs and of its operands at the 57 GB/s a CU takes in, a
 //     workgroup a fixed part that grows with its tile (prologue and epilogue),
 //     blocks run in rounds of 256 (one per CU), the weights stream at most at

@@ -28,18 +28,20 @@ from decide_amd import hip  # noqa: E402
 from decide_amd.hip import DeviceArray, Event, Stream  # noqa: E402
 from decide_amd.kernels import Epilogue, Kernels, fill_normal_f16, variants  # noqa: E402
 
-# decide's engine GEMM shapes (K, N) (gemm_configs.rs:385) plus BASELINE's Q/K/V group and
-# the un-interleaved MLP half, with the epilogue each runs under in the forward.
+PLAIN, NORM = False, True  # dh_gemm_nt, or dh_gemm_add_rmsnorm with the row norm that follows
+# decide's engine GEMM shapes (K, N) (gemm_configs.rs:385) plus a Q/K/V group and the un-interleaved MLP half, with the
+# epilogue each runs under in the forward and the calls it is timed as (their mean where there are two): a split K's
+# partials are summed by another kernel where a norm follows.
 ENGINE_SHAPES = [
-    (2560, 12352, Epilogue.StoreF32),  # GDN in-projection qkv|z|b|a
-    (2560, 10240, Epilogue.StoreF32),  # attention in-projection q|gate|k|v
-    (2560, 18432, Epilogue.SwigluF16),  # MLP gate|up
-    (4096, 2560, Epilogue.AddF32),  # attention / GDN out-projection
-    (9216, 2560, Epilogue.AddF32),  # MLP down
-    (2560, 2048, Epilogue.StoreF32),  # pruned layer k|v
-    (2560, 8192, Epilogue.StoreF32),  # pruned layer q|gate
-    (2560, 6144, Epilogue.StoreF32),  # BASELINE attention group Q|K|V
-    (2560, 9216, Epilogue.StoreF32),
+    (2560, 12352, Epilogue.StoreF32, (PLAIN,)),  # GDN in-projection qkv|z|b|a
+    (2560, 10240, Epilogue.StoreF32, (PLAIN,)),  # attention in-projection q|gate|k|v
+    (2560, 18432, Epilogue.SwigluF16, (PLAIN,)),  # MLP gate|up
+    (4096, 2560, Epilogue.AddF32, (NORM,)),  # attention / GDN out-projection: the MLP's norm always follows
+    (9216, 2560, Epilogue.AddF32, (PLAIN, NORM)),  # MLP down: the next layer's norm follows, none after the last
+    (2560, 2048, Epilogue.StoreF32, (PLAIN,)),  # pruned layer k|v
+    (2560, 8192, Epilogue.StoreF32, (PLAIN,)),  # pruned layer q|gate
+    (2560, 6144, Epilogue.StoreF32, (PLAIN,)),  # attention group Q|K|V
+    (2560, 9216, Epilogue.StoreF32, (PLAIN,)),  # gate or up alone
 ]
 DEFAULT_MS = [1, 3, 8, 12, 16, 20, 24, 28, 32, 40, 48, 56, 64, 80, 96, 112, 128, 144, 163, 176, 200, 230, 256, 276, 320,
               370, 430, 490, 550, 603, 680, 760, 850, 950, 1024, 1150, 1300, 1500, 1700, 1900, 2100, 2307]
@@ -68,7 +70,7 @@ def main():
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
     ap.add_argument("--out", default="gpurun_out/tune_gemm.json")
     ap.add_argument("--ms", default=",".join(map(str, DEFAULT_MS)))
-    ap.add_argument("--shapes", default="", help="K:N pairs (default: the engine shapes)")
+    ap.add_argument("--shapes", default="", help="K:N pairs (default: the engine shapes); others run with StoreF32")
     ap.add_argument("--iters", type=int, default=12)
     args = ap.parse_args()
     if not hip.available():
@@ -76,8 +78,9 @@ def main():
     ms = [int(v) for v in args.ms.split(",") if v]
     shapes = ENGINE_SHAPES
     if args.shapes:
-        want = {tuple(int(x) for x in kv.split(":")) for kv in args.shapes.split(",")}
-        shapes = [s for s in ENGINE_SHAPES if (s[0], s[1]) in want]
+        engine = {(s[0], s[1]): s for s in ENGINE_SHAPES}
+        want = [tuple(int(x) for x in kv.split(":")) for kv in args.shapes.split(",")]
+        shapes = [engine.get(kn, (*kn, Epilogue.StoreF32, (PLAIN,))) for kn in want]
     k = Kernels()
     st = Stream()
     s = st.handle
@@ -88,34 +91,46 @@ def main():
     fill_normal_f16(k.ctx, s, (x, 0), maxm * maxk, 8, 1.0)
     y = DeviceArray((maxm * maxn,), np.float32)
     y.zero_()
+    h = DeviceArray((maxm * maxn,), np.float16)
+    norm_w = DeviceArray((maxn,), np.float32)
+    norm_w.zero_()
     k.gemm.warm_up(s, maxm)
     st.synchronize()
     nvar = len(variants())
     # Let the clocks settle first: the first ~300 launches of sustained MFMA load run ~10 % slower.
-    kk0, n0, epi0 = shapes[0]
+    kk0, n0, epi0, _ = shapes[0]
     for i in range(400):
         k.gemm.gemm(s, (x, 0), (pool, 0), (y, 0), max(ms), n0, kk0, kk0, kk0, n0 // 2 if epi0 == Epilogue.SwigluF16 else n0,
                     epi0)
     st.synchronize()
     results = []
     t_start = time.time()
-    for (kk, n, epi) in shapes:
+    for (kk, n, epi, forms) in shapes:
         wbytes = n * kk * 2
         copies = max(1, min(POOL_BYTES // wbytes, (400 << 20) // wbytes + 1))
         ldy = n // 2 if epi == Epilogue.SwigluF16 else n
         for m in ms:
+            def call(i, norm):
+                w = (pool, (i % copies) * wbytes)
+                if norm:
+                    k.gemm.gemm_add_rmsnorm(s, (x, 0), w, (y, 0), m, n, kk, kk, kk, ldy, (norm_w, 0), (h, 0), n)
+                else:
+                    k.gemm.gemm(s, (x, 0), w, (y, 0), m, n, kk, kk, kk, ldy, epi)
+
             def timeit():
-                for i in range(3):
-                    k.gemm.gemm(s, (x, 0), (pool, (i % copies) * wbytes), (y, 0), m, n, kk, kk, kk, ldy, epi)
-                e0, e1 = Event(), Event()
-                e0.record(s)
-                for i in range(args.iters):
-                    k.gemm.gemm(s, (x, 0), (pool, (i % copies) * wbytes), (y, 0), m, n, kk, kk, kk, ldy, epi)
-                e1.record(s)
-                e1.synchronize()
-                t = e0.elapsed_ms(e1) / args.iters * 1e3
-                e0.destroy()
-                e1.destroy()
+                t = 0.0
+                for norm in forms:
+                    for i in range(3):
+                        call(i, norm)
+                    e0, e1 = Event(), Event()
+                    e0.record(s)
+                    for i in range(args.iters):
+                        call(i, norm)
+                    e1.record(s)
+                    e1.synchronize()
+                    t += e0.elapsed_ms(e1) / args.iters * 1e3 / len(forms)
+                    e0.destroy()
+                    e1.destroy()
                 return t
             rows = []
             for v in range(nvar):
@@ -139,7 +154,7 @@ def main():
             fl = 2.0 * m * n * kk
             rec = {"k": kk, "n": n, "m": m, "epi": int(epi), "best": [v, sp, round(t, 2)],
                    "planner": [plan["variant"], plan["splits"], round(t_plan, 2)],
-                   "tflops_best": round(fl / t / 1e6, 1), "top": [[round(a, 2), b, c] for a, b, c in rows[:6]]}
+                   "tflops_best": round(fl / t / 1e6, 1), "top": [[round(a, 2), b, c] for a, b, c in rows[:7]]}
             results.append(rec)
             print(json.dumps(rec), flush=True)
     os.makedirs(os.path.dirname(args.out) or ".", exist_ok=True)
