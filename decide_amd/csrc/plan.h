@@ -25,9 +25,12 @@ struct Plan {
 // output columns per workgroup, M <= 16, K a multiple of 128.
 constexpr int kStreamVariant = 64;  // DH_GEMM_STREAM_VARIANT
 constexpr uint32_t kStreamMaxM = 16;
-// Widest N (summed over a grouped launch's members) the streaming kernel takes:
-// measured faster than the FM = 1/2 tile variants with split-K up to here
-// (k|v, o and down of the pruned layer) and slower beyond (q|gate, gate|up).
+// Widest N (summed over a grouped launch's members) the streaming kernel takes, where the table has no choice of its
+// own. Against the best split of the 32 x 96 tile, weights from HBM, 1 to 16 rows: k|v (2560 -> 2048) 9.2-10.6 us
+// streaming, 9.5-10.1 tiled, so it streams; out (4096 -> 2560) 12.0-12.9 against 10.7-11.4 and down (9216 -> 2560)
+// 15.7-17.5 against 14.9-15.3, so the table's tiles take them. Of other shapes, N = 1024 to 4096 at 3 and 12 rows, the
+// best split of that tile is level to 25 % ahead, but the cost model does not find it (1024 -> 1024 at 17 rows: eight
+// splits, 9.1 us; streaming at 12 rows 7.8; best split 6.4), so they stream. Wider N (q|gate, gate|up) streams slower.
 constexpr uint32_t kStreamMaxN = 4096;
 
 // Model estimate for one (variant, splits) choice; +inf if the choice is not

@@ -186,6 +186,19 @@ def test_planner_has_no_row_count_of_its_own(m):
     assert len({(p["variant"], p["splits"]) for p in plans}) == 1, plans
 
 
+@pytest.mark.parametrize("m", range(1, 17))
+def test_planner_reaches_its_rows_for_few_rows(m):
+    """Up to 16 rows the table comes before the weight-streaming kernel: out and down take the 32 x 96 tile it holds for
+    them (about 1 us faster), k|v below 16 rows and shapes the table does not hold stream."""
+    tile = next(i for i, v in enumerate(variants()) if (v["bm"], v["bn"]) == (32, 96))
+    for k in (4096, 9216):
+        p = plan_for(m, 2560, k, Epilogue.AddF32)
+        assert p["variant"] == tile and p["splits"] > 1, p
+    for n, k in ((2048, 2560), (2560, 2560), (4096, 4096)):
+        p = plan_for(m, n, k, Epilogue.StoreF32)
+        assert p["variant"] == _lib.DH_GEMM_STREAM_VARIANT or (m == 16 and n == 2048), p
+
+
 def test_tile_order_gives_each_xcd_a_compact_block():
     """The 8 XCDs each take a contiguous run of work ids. At M = 2,307 the down and out projections make
     15 x 16 tiles of 160 x 160 (30 per XCD): in M-fastest order each XCD's run covers all 15 row blocks of X

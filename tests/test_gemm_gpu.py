@@ -66,7 +66,7 @@ def test_small_shapes_planner(gpu, kernels, stream, m, n, k, epi):
 
 
 # the weight-streaming kernel (M <= 16, K % 128 == 0): split-K and single-pass shapes, ragged M, N tails
-STREAM = [(1, 32, 128), (3, 2560, 9216), (16, 4096, 2560), (7, 96, 384), (16, 64, 1024), (13, 2048, 2560),
+STREAM = [(1, 32, 128), (3, 2560, 8192), (16, 4096, 2560), (7, 96, 384), (16, 64, 1024), (13, 2048, 2560),
           (2, 160, 4096)]
 
 

@@ -181,6 +181,52 @@ def test_gated_delta_blocks_keep_a_bad_token_to_itself_and_later_ones(gpu, kerne
     assert not np.isfinite(want[0]).all()
 
 
+@pytest.mark.parametrize("what", ["fast decay", "gates past the clamp", "one key, beta 1, no decay"])
+def test_gated_delta_blocks_with_extreme_gates(gpu, kernels, stream, what):
+    """The block kernel (t = 45: two whole blocks and one of 13) against the oracle where its γ ratios underflow
+    (g ≈ e^-37 per token), where log g passes the clamp that keeps differences of -inf out of them (a = 1e5 and inf at a
+    few tokens: g = 0), and with every key the same, beta = 1 and g = 1, where A is all ones and a series of its powers
+    would cancel. Bound as in test_gated_delta_blocks_match_oracle."""
+    t = 45
+    q, k, v, p, a_log, dt_bias, s0 = _delta_inputs(t, 310, a_log_std=0.0)
+    if what == "fast decay":
+        a_log[:], dt_bias[:], p[:, LIN_A:LIN_A + NV] = 2.0, 0.0, 5.0
+    elif what == "gates past the clamp":
+        p[[3, 18, 32], LIN_A:LIN_A + NV] = 1e5
+        p[[16, 31, 40], LIN_A:LIN_A + NV] = np.inf
+    else:
+        k[:] = k[0] / np.linalg.norm(k[0], axis=-1, keepdims=True)
+        a_log[:], p[:, LIN_B:LIN_B + NV] = -np.inf, 50.0
+    o, s1 = _run_delta(kernels, stream, q, k, v, p, a_log, dt_bias, s0, t)
+    wo, ws = orc.gated_delta(q, k, v, p[:, LIN_A:LIN_A + NV], p[:, LIN_B:LIN_B + NV], a_log, dt_bias, s0, t)
+    assert np.isfinite(o).all() and np.isfinite(s1).all() and np.isfinite(wo).all()
+    assert orc.rel_frobenius(o, wo) <= 2e-6, orc.rel_frobenius(o, wo)
+    assert orc.rel_frobenius(s1, ws) <= 2e-6, orc.rel_frobenius(s1, ws)
+
+
+def test_gated_delta_blocks_carry_state_and_leave_it_unwritten(gpu, kernels, stream):
+    """Two calls of the block kernel, in place, the second from the first's state, against the oracle over all tokens;
+    and a call with write_state = 0, whose state_out may be null, gives the same outputs and writes no state."""
+    t1, t2 = 39, 45
+    q, k, v, p, a_log, dt_bias, s0 = _delta_inputs(t1 + t2, 330)
+    wo, ws = orc.gated_delta(q, k, v, p[:, LIN_A:LIN_A + NV], p[:, LIN_B:LIN_B + NV], a_log, dt_bias, s0, t1 + t2)
+    o1, s_mid = _run_delta(kernels, stream, q[:t1], k[:t1], v[:t1], p[:t1], a_log, dt_bias, s0, t1, in_place=True)
+    rest = (q[t1:], k[t1:], v[t1:], p[t1:], a_log, dt_bias, s_mid, t2)
+    o2, s_end = _run_delta(kernels, stream, *rest, in_place=True)
+    assert orc.rel_frobenius(np.concatenate([o1, o2]), wo) <= 2e-6
+    assert orc.rel_frobenius(s_end, ws) <= 2e-6
+    o3, untouched = _run_delta(kernels, stream, *rest, write=False)
+    np.testing.assert_array_equal(o3, o2)
+    assert np.isnan(untouched).all(), "write_state = 0 must leave state_out untouched"
+    qd, kd, vd, pd, sd = (to_dev(x) for x in (*rest[:4], s_mid))
+    o4 = empty((t2, NV, DV), np.float32)
+    kernels.delta.gated_delta(stream, (qd, 0), (kd, 0), (vd, 0), (pd, LIN_A * 4), (pd, LIN_B * 4), (to_dev(a_log), 0),
+                              (to_dev(dt_bias), 0), (sd, 0), (0, 0), (o4, 0), t2, LIN_IN_N, False)
+    sync()
+    np.testing.assert_array_equal(to_host(o4), o2)
+    np.testing.assert_array_equal(to_host(sd), s_mid)
+
+
 @pytest.mark.parametrize("impl", ["chunked", "sequential"])
 def test_gated_delta_unit_gate_known_answer(gpu, kernels_delta_sequential, kernels_delta_chunked, stream, impl):
     """decide's known answer (cpu_ref.rs:224-236) through both GPU implementations: one step, beta = 1 (b = 50),
