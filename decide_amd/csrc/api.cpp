@@ -172,11 +172,11 @@ int check_gemm(const dh_ctx* c, const void* x, uint32_t ldx, const void* w, uint
   return check_gemm_fast(x, ldx, w, ldw, y, ldy, m, n, k, epi);
 }
 
-dh::Plan choose_plan(const dh_ctx* c, uint32_t m, uint32_t n, uint32_t k, uint32_t epi) {
+dh::Plan choose_plan(const dh_ctx* c, uint32_t m, uint32_t n, uint32_t k) {
   int fv;
   uint32_t fs;
-  if (forced_plan(c, &fv, &fs)) return dh::plan_make(fv, std::max(1u, fs), m, n, k, epi);
-  return dh::plan_gemm(m, n, k, epi, c ? c->ws_cap : (512ull << 20));
+  if (forced_plan(c, &fv, &fs)) return dh::plan_make(fv, std::max(1u, fs), m, n, k);
+  return dh::plan_gemm(m, n, k, c ? c->ws_cap : (512ull << 20));
 }
 
 // Enqueues plan p. Split-K partials go to `fixed_ws` when given (it must hold
@@ -310,7 +310,7 @@ int dh_gemm_nt(dh_ctx* ctx, void* stream, const void* x, uint32_t ldx, const voi
                                                 epi, s),
                       "gemm reference kernel launch");
   }
-  const dh::Plan p = choose_plan(ctx, m, n, k, epi);
+  const dh::Plan p = choose_plan(ctx, m, n, k);
   if (p.variant < 0) return fail(DH_EINVAL, "gemm: no plan for M = %u, N = %u, K = %u", m, n, k);
   dh_gemm_member mem{w, y, ldw, ldy, n, epi};
   return launch_plan(ctx, s, p, x, ldx, m, k, &mem, 1);
@@ -327,7 +327,7 @@ int dh_gemm_add_rmsnorm(dh_ctx* ctx, void* stream, const void* x, uint32_t ldx, 
   if (m && (!norm_w || !h)) return fail(DH_EINVAL, "gemm_add_rmsnorm: null norm weight or output");
   hipStream_t s = (hipStream_t)stream;
   if (!(ctx->flags & DH_GEMM_REFERENCE) && m && k) {
-    const dh::Plan p = choose_plan(ctx, m, n, k, DH_EPI_ADD_F32);
+    const dh::Plan p = choose_plan(ctx, m, n, k);
     if (p.variant >= 0 && p.splits > 1 && dh::splitk_add_rmsnorm_fits(p.splits, n, ldy, ldh, y, norm_w, h)) {
       dh_gemm_member mem{w, y, ldw, ldy, n, DH_EPI_ADD_F32};
       const float* partials = nullptr;
@@ -367,8 +367,8 @@ int dh_gemm_nt_noalloc(dh_ctx* ctx, void* stream, const void* x, uint32_t ldx, c
   }
   int fv;
   uint32_t fs;
-  const dh::Plan p = forced_plan(ctx, &fv, &fs) ? dh::plan_make(fv, std::max(1u, fs), m, n, k, epi)
-                                                : dh::plan_gemm(m, n, k, epi, dh::kNoAllocScratchBytes);
+  const dh::Plan p = forced_plan(ctx, &fv, &fs) ? dh::plan_make(fv, std::max(1u, fs), m, n, k)
+                                                : dh::plan_gemm(m, n, k, dh::kNoAllocScratchBytes);
   if (p.variant < 0) return fail(DH_EINVAL, "gemm (no-alloc): no plan for M = %u, N = %u, K = %u", m, n, k);
   if (p.ws_bytes > dh::kNoAllocScratchBytes)
     return fail(DH_EINVAL,
@@ -410,7 +410,7 @@ int dh_gemm_nt_grouped(dh_ctx* ctx, void* stream, const void* x, uint32_t ldx, u
   }
   int fv;
   uint32_t fs;
-  dh::Plan p = forced_plan(ctx, &fv, &fs) ? dh::plan_make(fv, 1, m, n_total, k, 0u) : dh::plan_grouped(m, k, ns, count);
+  dh::Plan p = forced_plan(ctx, &fv, &fs) ? dh::plan_make(fv, 1, m, n_total, k) : dh::plan_grouped(m, k, ns, count);
   if (p.variant < 0) return fail(DH_EINVAL, "gemm grouped: no plan");
   return launch_plan(ctx, s, p, x, ldx, m, k, members, count);
 }
@@ -420,7 +420,7 @@ static_assert(dh::kStreamVariant == (int)DH_GEMM_STREAM_VARIANT, "the streaming 
 int dh_gemm_plan_for(const dh_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint32_t epi, dh_gemm_plan* out) {
   if (!out) return fail(DH_EINVAL, "dh_gemm_plan_for: out is NULL");
   if (epi > 3u || m < 1 || n % 32 || k % 32) return fail(DH_EINVAL, "dh_gemm_plan_for: invalid shape");
-  const dh::Plan p = choose_plan(ctx, m, n, k, epi);
+  const dh::Plan p = choose_plan(ctx, m, n, k);
   if (p.variant < 0) return fail(DH_EINVAL, "dh_gemm_plan_for: no plan");
   out->variant = (uint32_t)p.variant;
   if (p.variant == dh::kStreamVariant) {
@@ -514,7 +514,7 @@ int dh_warm_up(dh_ctx* ctx, void* stream, uint32_t max_m) {
   for (int v = 0; v < dh::variant_count() && rc == DH_OK; ++v) {
     const dh::VariantInfo vi = dh::variant_info(v);
     dh_gemm_member mem{base + xb, base + xb + wb, 64, (uint32_t)vi.bn(), (uint32_t)vi.bn(), DH_EPI_STORE_F32};
-    rc = launch_plan(ctx, s, dh::plan_make(v, 1, 16, vi.bn(), 64, 0u), base, 64, 16, 64, &mem, 1);
+    rc = launch_plan(ctx, s, dh::plan_make(v, 1, 16, vi.bn(), 64), base, 64, 16, 64, &mem, 1);
   }
   if (rc == DH_OK) {
     dh_gemm_member mem{base + xb, base + xb + wb, 128, 32, 32, DH_EPI_STORE_F32};
@@ -524,7 +524,7 @@ int dh_warm_up(dh_ctx* ctx, void* stream, uint32_t max_m) {
     // and the split-K reduction once (two splits of K = 128)
     const dh::VariantInfo vi = dh::variant_info(0);
     dh_gemm_member mem{base + xb, base + xb + wb, 128, (uint32_t)vi.bn(), (uint32_t)vi.bn(), DH_EPI_STORE_F32};
-    rc = launch_plan(ctx, s, dh::plan_make(0, 2, 8, vi.bn(), 128, 0u), base, 128, 8, 128, &mem, 1);
+    rc = launch_plan(ctx, s, dh::plan_make(0, 2, 8, vi.bn(), 128), base, 128, 8, 128, &mem, 1);
   }
   if (rc == DH_OK) {
     e = hipStreamSynchronize(s);

@@ -194,7 +194,7 @@ const Measured kMeasured[] = {
 };
 }  // namespace
 
-Plan plan_make(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k, uint32_t epi) {
+Plan plan_make(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k) {
   const VariantInfo v = variant_info(variant);
   Plan p{};
   p.variant = variant;
@@ -229,7 +229,7 @@ double plan_estimate_us(int variant, uint32_t splits, uint32_t m, uint32_t n, ui
 }
 
 namespace {
-Plan plan_model(uint32_t m, uint32_t n, uint32_t k, uint32_t epi, uint64_t max_ws) {
+Plan plan_model(uint32_t m, uint32_t n, uint32_t k, uint64_t max_ws) {
   Plan best{};
   best.est_us = std::numeric_limits<double>::infinity();
   best.variant = -1;
@@ -237,7 +237,7 @@ Plan plan_model(uint32_t m, uint32_t n, uint32_t k, uint32_t epi, uint64_t max_w
     for (uint32_t s : kSplitMenu) {
       const double t = plan_estimate_us(v, s, m, n, k);
       if (!(t < best.est_us)) continue;
-      const Plan p = plan_make(v, s, m, n, k, epi);
+      const Plan p = plan_make(v, s, m, n, k);
       if (p.ws_bytes > max_ws) continue;
       best = p;
     }
@@ -272,10 +272,10 @@ Plan plan_stream(uint32_t m, uint32_t n, uint32_t k, uint64_t max_ws) {
   return p;
 }
 
-Plan plan_gemm(uint32_t m, uint32_t n, uint32_t k, uint32_t epi, uint64_t max_ws) {
+Plan plan_gemm(uint32_t m, uint32_t n, uint32_t k, uint64_t max_ws) {
   // decide's contract admits N = 0 (nothing to launch: an empty grid) and K = 0 (the tiles run no
   // stage and store the empty sum).
-  if (n == 0 || k == 0) return plan_make(0, 1, m, n, k, epi);
+  if (n == 0 || k == 0) return plan_make(0, 1, m, n, k);
   const Measured* best = nullptr;
   double best_us = std::numeric_limits<double>::infinity();
   for (const Measured& e : kMeasured) {
@@ -294,15 +294,14 @@ Plan plan_gemm(uint32_t m, uint32_t n, uint32_t k, uint32_t epi, uint64_t max_ws
       best = &e;
     }
   }
-  if (best) return plan_make(best->variant, best->splits, m, n, k, epi);
+  if (best) return plan_make(best->variant, best->splits, m, n, k);
   if (m <= kStreamMaxM && n <= kStreamMaxN && k % 128 == 0 && n % 32 == 0) return plan_stream(m, n, k, max_ws);
-  return plan_model(m, n, k, epi, max_ws);
+  return plan_model(m, n, k, max_ws);
 }
 
 uint64_t plan_ws_need(uint32_t max_m, uint32_t n, uint32_t k, uint64_t max_ws) {
   uint64_t need = 0;
-  for (uint32_t m = 1; m <= max_m; ++m)
-    for (uint32_t epi = 0; epi < 4; ++epi) need = std::max(need, plan_gemm(m, n, k, epi, max_ws).ws_bytes);
+  for (uint32_t m = 1; m <= max_m; ++m) need = std::max(need, plan_gemm(m, n, k, max_ws).ws_bytes);
   return need;
 }
 
@@ -314,7 +313,7 @@ Plan plan_grouped(uint32_t m, uint32_t k, const uint32_t* ns, uint32_t count) {
   // stripes member by member.
   uint32_t n_total = 0;
   for (uint32_t i = 0; i < count; ++i) n_total += ns[i];
-  const Plan p = plan_gemm(m, n_total, k, 0u, 0);
+  const Plan p = plan_gemm(m, n_total, k, 0);
   if (p.variant == kStreamVariant) return p;
   // the width whose single-GEMM stripe count equals the grouped one for variant v
   auto grouped_n = [&](int v) {
@@ -332,7 +331,7 @@ Plan plan_grouped(uint32_t m, uint32_t k, const uint32_t* ns, uint32_t count) {
     const double t = plan_estimate_us(v, 1, m, grouped_n(v), k);
     if (t < best_us) {
       best_us = t;
-      best = plan_make(v, 1, m, n_total, k, 0u);
+      best = plan_make(v, 1, m, n_total, k);
     }
   }
   return best;

@@ -1,4 +1,5 @@
-// GEMM launch planner for MI355X: (m, n, k, epi) → tile variant + split-K.
+// GEMM launch planner for MI355X: (m, n, k) → tile variant + split-K, for every
+// epilogue alike.
 // decide's counterpart is gemm_configs::plan / recommend
 // (crates/decide-metal/src/gemm_configs.rs:290-314), a table measured on an
 // M1 Pro. This one is a table measured on an MI355X for decide's engine
@@ -37,13 +38,13 @@ constexpr uint32_t kStreamMaxN = 4096;
 // valid for the shape.
 double plan_estimate_us(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k);
 // Builds the plan for (variant, splits), filling the derived fields.
-Plan plan_make(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k, uint32_t epi);
+Plan plan_make(int variant, uint32_t splits, uint32_t m, uint32_t n, uint32_t k);
 // The weight-streaming kernel's plan (M <= kStreamMaxM, K % 128 == 0, N % 32 == 0).
 Plan plan_stream(uint32_t m, uint32_t n, uint32_t k, uint64_t max_ws);
 // Best plan for a single GEMM. `max_ws` caps the split-K workspace bytes.
-Plan plan_gemm(uint32_t m, uint32_t n, uint32_t k, uint32_t epi, uint64_t max_ws);
-// The largest split-K workspace plan_gemm asks for over every M in 1..max_m and
-// every epilogue at (n, k): the workspace a caller must hold so that no call of
+Plan plan_gemm(uint32_t m, uint32_t n, uint32_t k, uint64_t max_ws);
+// The largest split-K workspace plan_gemm asks for over every M in 1..max_m at
+// (n, k): the workspace a caller must hold so that no call of
 // up to max_m rows grows it. The table switches split counts between measured
 // rows, so the need is not monotone in M; this sweeps every M.
 uint64_t plan_ws_need(uint32_t max_m, uint32_t n, uint32_t k, uint64_t max_ws);

@@ -176,7 +176,7 @@ int dh_gemm_plan_for(const dh_ctx* ctx, uint32_t m, uint32_t n, uint32_t k, uint
 /* The split-K workspace (bytes) that dh_gemm_nt's planner asks for at its
  * largest over every m in 1..max_m and every epilogue at (n, k), on this
  * context (no device needed; the planner runs once per m, so max_m is capped
- * at DH_PLAN_MAX_ROWS, about 0.3 s of host time per shape there). dh_warm_up
+ * at DH_PLAN_MAX_ROWS, about 0.15 s of host time per shape there). dh_warm_up
  * holds at least this for decide's engine shapes; a caller with other shapes
  * can size its own calls with it. */
 int dh_gemm_ws_need(const dh_ctx* ctx, uint32_t max_m, uint32_t n, uint32_t k, uint64_t* out);
