@@ -219,6 +219,49 @@ __global__ __launch_bounds__(32 * KV) void rmsnorm_rows_vec_kernel(const float* 
   }
 }
 
+// The same norm, the same bits, with a wave per two rows and eight rows per workgroup: the weights are loaded once for
+// both rows and both rows' loads are in flight together. For many rows, where every CU has work either way and a
+// workgroup's barriers and idle threads count instead.
+template <int KV>
+__global__ __launch_bounds__(256) void rmsnorm_rows_pair_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                _Float16* __restrict__ y,
+                                                                const uint32_t* __restrict__ rowmap, uint32_t rows,
+                                                                uint32_t h, uint32_t ld_in, uint32_t ld_out,
+                                                                uint32_t add_one, float eps) {
+  const uint32_t row0 = 2 * (blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (row0 >= rows) return;
+  const uint32_t lane = threadIdx.x & 63, n4 = h / 4;
+  const bool two = row0 + 1 < rows;
+  const float* xr0 = x + (size_t)(rowmap ? rowmap[row0] : row0) * ld_in;
+  const float* xr1 = two ? x + (size_t)(rowmap ? rowmap[row0 + 1] : row0 + 1) * ld_in : xr0;
+  f4 v0[KV], v1[KV], wv[KV];
+#pragma unroll
+  for (int q = 0; q < KV; ++q) {
+    const uint32_t i = lane + 64 * q;
+    v0[q] = i < n4 ? *(const f4*)(xr0 + 4 * i) : f4{0.f, 0.f, 0.f, 0.f};
+    v1[q] = i < n4 ? *(const f4*)(xr1 + 4 * i) : f4{0.f, 0.f, 0.f, 0.f};
+    wv[q] = i < n4 ? weight4(w, i, add_one) : f4{0.f, 0.f, 0.f, 0.f};
+  }
+  float ss0 = 0.f, ss1 = 0.f;
+#pragma unroll
+  for (int q = 0; q < KV; ++q) {
+    ss0 += sq4(v0[q]);
+    ss1 += sq4(v1[q]);
+  }
+  const float inv0 = rsqrtf(wave_sum(ss0) / (float)h + eps);
+  const float inv1 = rsqrtf(wave_sum(ss1) / (float)h + eps);
+  _Float16* yr0 = y + (size_t)row0 * ld_out;
+  _Float16* yr1 = yr0 + ld_out;
+#pragma unroll
+  for (int q = 0; q < KV; ++q) {
+    const uint32_t i = lane + 64 * q;
+    if (i < n4) {
+      *(h4*)(yr0 + 4 * i) = norm4w(v0[q], inv0, wv[q]);
+      if (two) *(h4*)(yr1 + 4 * i) = norm4w(v1[q], inv1, wv[q]);
+    }
+  }
+}
+
 // The residual add of a split-K projection fused with the norm that follows it:
 //   x[r] += Σ_s ws[s][r]   (the partials summed in split order, then added to the row: splitk_reduce_kernel's AddF32)
 //   y[r] = half(x[r] · rsqrt(mean(x[r]²) + eps) · w')   (rmsnorm_rows_vec_kernel<KV>'s arithmetic)
@@ -314,16 +357,31 @@ hipError_t launch_rmsnorm_rows(const float* x, const float* w, _Float16* y, cons
   const bool vec = h % 4 == 0 && h <= 256 * 16 && ld_in % 4 == 0 && ld_out % 4 == 0 && (uintptr_t)x % 16 == 0 &&
                    (uintptr_t)w % 16 == 0 && (uintptr_t)y % 8 == 0;
   if (vec) {
+    // A workgroup per row, or a wave per two rows from kManyRows on. Workgroup against wave, 2,307 rows: 2,560 columns
+    // 6.6 and 7.2 us, 3,072 9.2 and 8.8; 2,700 rows: 1,536 columns 6.3 and 5.4, 2,560 8.8 and 8.2, 4,096 12.8 and 12.4;
+    // 4,000 rows: 2,560 columns 12.7 and 11.1, 3,072 14.5 and 12.7; 16,000 rows of 516 20.5 and 11.9. One wave per row
+    // up to 512 columns stays ahead (16,000 rows of 512 9.9 and 10.9), as do wider rows than 2,560 past kManyWideRows
+    // (5,000 rows of 4,096 20.5 and 23.6, of 3,072 17.1 and 18.2).
+    constexpr uint32_t kManyRows = 2400, kManyWideRows = 4400;
+    const bool pairs = h > 256 * 2 && rows > kManyRows && (h <= 256 * 10 || rows <= kManyWideRows);
+    const uint32_t threads = pairs ? 256 : h <= 256 * 2 ? 64 : h <= 256 * 10 ? 320 : 512;
     // a launch holds fewer than 2^32 threads: more rows than that go in several
-    const uint32_t threads = h <= 256 * 2 ? 64 : h <= 256 * 10 ? 320 : 512, most = UINT32_MAX / threads;
-    const auto kernel = h <= 256 * 2    ? rmsnorm_rows_vec_kernel<2>
-                        : h <= 256 * 10 ? rmsnorm_rows_vec_kernel<10>
-                                        : rmsnorm_rows_vec_kernel<16>;
+    const uint64_t most = (uint64_t)(UINT32_MAX / threads) * (pairs ? 8 : 1);
+    const uint32_t one = add_one ? 1u : 0u;
     for (uint32_t r0 = 0; r0 < rows;) {
-      const uint32_t n = std::min(most, rows - r0);
-      hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), 0, s, rowmap ? x : x + (size_t)r0 * ld_in, w,
-                         y + (size_t)r0 * ld_out, rowmap ? rowmap + r0 : nullptr, h, ld_in, ld_out, add_one ? 1u : 0u,
-                         eps);
+      const uint32_t n = (uint32_t)std::min<uint64_t>(most, rows - r0);
+      const float* xs = rowmap ? x : x + (size_t)r0 * ld_in;
+      _Float16* ys = y + (size_t)r0 * ld_out;
+      const uint32_t* map = rowmap ? rowmap + r0 : nullptr;
+      if (pairs)
+        hipLaunchKernelGGL(h <= 256 * 10 ? rmsnorm_rows_pair_kernel<10> : rmsnorm_rows_pair_kernel<16>,
+                           dim3((uint32_t)(((uint64_t)n + 7) / 8)), dim3(threads), 0, s, xs, w, ys, map, n, h, ld_in,
+                           ld_out, one, eps);
+      else
+        hipLaunchKernelGGL(h <= 256 * 2    ? rmsnorm_rows_vec_kernel<2>
+                           : h <= 256 * 10 ? rmsnorm_rows_vec_kernel<10>
+                                           : rmsnorm_rows_vec_kernel<16>,
+                           dim3(n), dim3(threads), 0, s, xs, w, ys, map, h, ld_in, ld_out, one, eps);
       if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
       r0 += n;
     }

@@ -132,6 +132,26 @@ def test_rmsnorm_rows_at_the_edges_of_the_row_widths(gpu, kernels, stream, h):
     orc.assert_close(f"rmsnorm h{h}", got[:rows], orc.f16_round(orc.rmsnorm(x[rowmap], w, True)), atol=1e-3, rtol=2e-3)
 
 
+@pytest.mark.parametrize("h", [512, 516, 1024, 2556, 2560, 2564, 4096])
+@pytest.mark.parametrize("rows", [2401, 2402, 4400, 4401])
+def test_rmsnorm_of_many_rows_has_the_bits_of_few(gpu, kernels, stream, h, rows):
+    """From 2,401 rows on (to 4,400 for rows wider than 2,560) a wave takes two rows, the last one alone where the
+    count is odd: bit for bit what a call with a few of these rows gives, and nothing past the last row."""
+    x = synth.normal_f32(synth.seed_for(106), (rows, h), 2.0)
+    w = synth.normal_f32(synth.seed_for(107), (h,), 0.3)
+    rowmap = np.random.default_rng(h).permutation(rows).astype(np.uint32)
+    xd, wd = to_dev(x), to_dev(w)
+    y, few = full((rows + 1, h), np.float16, 7.0), full((600, h), np.float16, 7.0)
+    kernels.norm.rmsnorm(stream, (xd, 0), (wd, 0), (y, 0), (u32(rowmap), 0), rows, h, h, h, True)
+    kernels.norm.rmsnorm(stream, (xd, 0), (wd, 0), (few, 0), (u32(rowmap[-600:]), 0), 600, h, h, h, True)
+    sync()
+    got = to_host(y)
+    assert (got[rows] == 7.0).all()
+    np.testing.assert_array_equal(got[rows - 600:rows].view(np.uint16), to_host(few).view(np.uint16))
+    orc.assert_close(f"rmsnorm h{h}", got[:8].astype(np.float32), orc.f16_round(orc.rmsnorm(x[rowmap[:8]], w, True)),
+                     atol=1e-3, rtol=2e-3)
+
+
 def test_rmsnorm_rows_of_more_threads_than_a_launch_holds(gpu, kernels, stream):
     """A launch holds fewer than 2^32 threads, 64 per row here: rows past that still come out."""
     rows, h = (2**32 // 64) + 3, 4
