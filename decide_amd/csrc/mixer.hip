@@ -442,10 +442,12 @@ __global__ void embed_bf16_kernel(const uint32_t* __restrict__ ids, const uint16
 hipError_t launch_embed_bf16(const uint32_t* ids, const uint16_t* table, float* out, uint32_t t, uint32_t h,
                              hipStream_t s) {
   if (t == 0) return hipSuccess;
-  // one workgroup per row, as many threads as it has 8-column pieces (2,307 rows of 2,560: 9.7 → 7.3 µs against two
-  // workgroups of 256)
-  const uint32_t threads = std::min<uint32_t>(1024, (h / 8 + 63) / 64 * 64);
-  hipLaunchKernelGGL(embed_bf16_kernel, dim3(1, t), dim3(threads), 0, s, ids, table, out, h);
+  // Up to 3,072 columns one workgroup per row, as many threads as it has 8-column pieces, beyond that workgroups of 256.
+  // One against several, 2,307 rows: 2,560 columns 7.2 and 9.6 us, 3,072 8.3 and 9.5, 4,096 10.8 and 10.2, 16,384 35.3
+  // and 33.6 (8,192 rows: 149 and 134).
+  const uint32_t pieces = (h / 8 + 63) / 64 * 64, threads = pieces <= 384 ? pieces : 256;
+  hipLaunchKernelGGL(embed_bf16_kernel, dim3((pieces + threads - 1) / threads, t), dim3(threads), 0, s, ids, table,
+                     out, h);
   return hipGetLastError();
 }
 
