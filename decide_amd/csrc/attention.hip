@@ -87,10 +87,11 @@ __device__ __forceinline__ s4 read_tr(const char* at) {
 }
 
 // The gate's σ: the hardware exp, and 1 / d from the hardware reciprocal (one ulp off at worst) and a Newton step, which
-// makes it the full division's value. For the 64 outputs of a lane the step takes 0.5 µs at 16 rows and 0.2 at 2,307, the
-// division 1.7 and 1.6. Past 2^100 d is held there (the step is inf · 0 at infinity; σ is 0 in fp16 by far).
+// makes it the full division's value. For the 64 outputs of a lane the step takes 0.3 µs at 16 rows, 2 at a single one
+// and none that shows from 32 on; the division took 1.7 at 16 and 1.6 at 2,307 rows. Past 2^100 d is held there (the step is inf · 0 at infinity; σ is 0 in fp16 by far).
 __device__ __forceinline__ float sigmoid(float x) {
-  const float e = 1.0f + __expf(-x), d = e > 0x1p100f ? 0x1p100f : e, r = __builtin_amdgcn_rcpf(d);
+  const float d = __builtin_elementwise_minimum(1.0f + __expf(-x), 0x1p100f);  // NaN stays NaN
+  const float r = __builtin_amdgcn_rcpf(d);
   return fmaf(fmaf(-d, r, 1.0f), r, r);
 }
 
