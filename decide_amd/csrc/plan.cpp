@@ -6,7 +6,10 @@
 //     (crates/decide-metal/src/gemm_configs.rs:247-283). `python -m
 //     decide_amd.tune_gemm` times the menu at these rows, as the calls the
 //     table's times are of; in a later run of it over all 378 points the
-//     table's choices were 1.2 % from that run's fastest;
+//     table's choices were 1.2 % from that run's fastest. Four rows more
+//     (800, 1400 and 1800 rows of the N = 2560 and 2048 shapes) cover ranges
+//     of 30 to 60 row counts where the choice between two of the 42 was 5-8 %
+//     behind; at 108 points between the rows it is 0.7 % behind on average;
 //   * a cost model for every other shape, fitted to the table's points (over
 //     the seven fastest choices of each in that later run: rms error 10 %, its
 //     pick 3.5 % from the fastest). Off the fit, 77 points of seven other
@@ -118,10 +121,11 @@ const Measured kMeasured[] = {
     {4096, 2560, 230, 20, 3, 18.6f}, {4096, 2560, 256, 20, 3, 19.2f}, {4096, 2560, 276, 20, 3, 19.9f},
     {4096, 2560, 320, 21, 4, 21.9f}, {4096, 2560, 370, 15, 3, 22.7f}, {4096, 2560, 430, 21, 3, 23.8f},
     {4096, 2560, 490, 21, 2, 26.2f}, {4096, 2560, 550, 21, 2, 27.2f}, {4096, 2560, 603, 14, 4, 28.4f},
-    {4096, 2560, 680, 10, 2, 30.9f}, {4096, 2560, 760, 10, 2, 32.3f}, {4096, 2560, 850, 8, 3, 36.2f},
-    {4096, 2560, 950, 4, 3, 38.1f}, {4096, 2560, 1024, 14, 2, 38.3f}, {4096, 2560, 1150, 14, 2, 40.0f},
-    {4096, 2560, 1300, 21, 1, 45.9f}, {4096, 2560, 1500, 10, 1, 50.8f}, {4096, 2560, 1700, 5, 2, 56.7f},
-    {4096, 2560, 1900, 5, 2, 59.0f}, {4096, 2560, 2100, 14, 1, 64.3f}, {4096, 2560, 2307, 14, 1, 65.5f},
+    {4096, 2560, 680, 10, 2, 30.9f}, {4096, 2560, 760, 10, 2, 32.3f}, {4096, 2560, 800, 14, 3, 32.5f},
+    {4096, 2560, 850, 8, 3, 36.2f}, {4096, 2560, 950, 4, 3, 38.1f}, {4096, 2560, 1024, 14, 2, 38.3f},
+    {4096, 2560, 1150, 14, 2, 40.0f}, {4096, 2560, 1300, 21, 1, 45.9f}, {4096, 2560, 1500, 10, 1, 50.8f},
+    {4096, 2560, 1700, 5, 2, 56.7f}, {4096, 2560, 1900, 5, 2, 59.0f}, {4096, 2560, 2100, 14, 1, 64.3f},
+    {4096, 2560, 2307, 14, 1, 65.5f},
     {9216, 2560, 1, 22, 8, 15.5f}, {9216, 2560, 3, 22, 8, 15.6f}, {9216, 2560, 8, 22, 8, 15.8f},
     {9216, 2560, 12, 22, 8, 15.9f}, {9216, 2560, 16, 22, 8, 15.9f}, {9216, 2560, 20, 22, 8, 15.9f},
     {9216, 2560, 24, 22, 8, 16.1f}, {9216, 2560, 28, 22, 8, 16.3f}, {9216, 2560, 32, 22, 8, 16.3f},
@@ -132,10 +136,11 @@ const Measured kMeasured[] = {
     {9216, 2560, 230, 20, 3, 28.2f}, {9216, 2560, 256, 19, 4, 29.6f}, {9216, 2560, 276, 3, 8, 31.2f},
     {9216, 2560, 320, 10, 4, 31.9f}, {9216, 2560, 370, 21, 3, 33.7f}, {9216, 2560, 430, 21, 3, 36.9f},
     {9216, 2560, 490, 4, 6, 40.0f}, {9216, 2560, 550, 14, 4, 41.1f}, {9216, 2560, 603, 14, 4, 42.2f},
-    {9216, 2560, 680, 10, 2, 48.3f}, {9216, 2560, 760, 4, 4, 49.5f}, {9216, 2560, 850, 8, 3, 56.9f},
-    {9216, 2560, 950, 5, 4, 60.5f}, {9216, 2560, 1024, 4, 3, 61.3f}, {9216, 2560, 1150, 14, 2, 65.0f},
-    {9216, 2560, 1300, 8, 2, 77.5f}, {9216, 2560, 1500, 4, 2, 82.7f}, {9216, 2560, 1700, 5, 2, 91.7f},
-    {9216, 2560, 1900, 5, 2, 97.4f}, {9216, 2560, 2100, 9, 2, 107.7f}, {9216, 2560, 2307, 14, 1, 115.3f},
+    {9216, 2560, 680, 10, 2, 48.3f}, {9216, 2560, 760, 4, 4, 49.5f}, {9216, 2560, 800, 14, 3, 50.8f},
+    {9216, 2560, 850, 8, 3, 56.9f}, {9216, 2560, 950, 5, 4, 60.5f}, {9216, 2560, 1024, 4, 3, 61.3f},
+    {9216, 2560, 1150, 14, 2, 65.0f}, {9216, 2560, 1300, 8, 2, 77.5f}, {9216, 2560, 1400, 9, 3, 79.5f},
+    {9216, 2560, 1500, 4, 2, 82.7f}, {9216, 2560, 1700, 5, 2, 91.7f}, {9216, 2560, 1900, 5, 2, 97.4f},
+    {9216, 2560, 2100, 9, 2, 107.7f}, {9216, 2560, 2307, 14, 1, 115.3f},
     {2560, 2048, 20, 22, 4, 8.4f}, {2560, 2048, 24, 22, 4, 8.5f}, {2560, 2048, 28, 22, 4, 8.6f},
     {2560, 2048, 32, 22, 3, 8.9f}, {2560, 2048, 40, 22, 4, 8.7f}, {2560, 2048, 48, 22, 4, 8.8f},
     {2560, 2048, 56, 18, 4, 9.9f}, {2560, 2048, 64, 22, 2, 9.8f}, {2560, 2048, 80, 22, 3, 9.4f},
@@ -147,8 +152,8 @@ const Measured kMeasured[] = {
     {2560, 2048, 603, 20, 1, 17.8f}, {2560, 2048, 680, 20, 1, 18.0f}, {2560, 2048, 760, 20, 1, 19.8f},
     {2560, 2048, 850, 20, 1, 20.0f}, {2560, 2048, 950, 20, 1, 20.4f}, {2560, 2048, 1024, 15, 1, 21.0f},
     {2560, 2048, 1150, 21, 1, 23.1f}, {2560, 2048, 1300, 15, 1, 22.8f}, {2560, 2048, 1500, 21, 1, 24.8f},
-    {2560, 2048, 1700, 21, 1, 27.2f}, {2560, 2048, 1900, 4, 2, 35.2f}, {2560, 2048, 2100, 14, 1, 33.5f},
-    {2560, 2048, 2307, 14, 1, 34.9f},
+    {2560, 2048, 1700, 21, 1, 27.2f}, {2560, 2048, 1800, 10, 1, 31.3f}, {2560, 2048, 1900, 4, 2, 35.2f},
+    {2560, 2048, 2100, 14, 1, 33.5f}, {2560, 2048, 2307, 14, 1, 34.9f},
     {2560, 8192, 1, 22, 2, 12.5f}, {2560, 8192, 3, 22, 2, 12.6f}, {2560, 8192, 8, 22, 2, 12.8f},
     {2560, 8192, 12, 22, 2, 13.2f}, {2560, 8192, 16, 22, 2, 13.3f}, {2560, 8192, 20, 22, 2, 13.9f},
     {2560, 8192, 24, 22, 2, 13.8f}, {2560, 8192, 28, 22, 2, 14.2f}, {2560, 8192, 32, 22, 2, 14.4f},
