@@ -7,14 +7,17 @@
 // Design (MI355X's own):
 //   * A workgroup is one kv head × 32 query rows; its 8 waves are the 4 query
 //     heads sharing that kv head × 2 halves of a staged tile of 64 keys, each
-//     wave taking all 32 rows on v_mfma_f32_32x32x16_f16. LDS bounds this
-//     kernel: a wave reads every K and Vᵀ fragment it multiplies, 32 KB per 32
-//     keys, so a fragment serves 32 rows. With 16 rows per wave and the waves
-//     split over rows instead of keys, 2,307 causal rows took 99 µs against 70,
-//     16 rows at position 2,000 92 against 53, 169 rows behind 107 keys 23.9
-//     against 19.9. The LDS reads and the products of 64 keys now take about
-//     2,050 clocks each, a tile about 3,200. The two key halves of a head meet
-//     once, at the end, through LDS: each wave takes half of the dims.
+//     wave taking all 32 rows on v_mfma_f32_32x32x16_f16. A wave reads every K
+//     and Vᵀ fragment it multiplies from LDS, 32 KB per 32 keys, so a fragment
+//     serves 32 rows. With 16 rows per wave and the waves split over rows
+//     instead of keys, 2,307 causal rows took 99 µs against 73, 16 rows at
+//     position 2,000 92 against 53, 169 rows behind 107 keys 24.0 against 20.0
+//     (and 8 rows at the start of a prompt 8.6 against 9.7). 64 keys are 64
+//     products of 32 clocks per SIMD, and as long in LDS reads at 128 bytes a
+//     clock; over 2,307 rows a tile takes 5,100 CU clocks, starts and ends
+//     included: the matrix cores are busy for 40 % of them, without a bank
+//     conflict. The two key halves of a head meet once, at the end, through
+//     LDS: each wave takes half of the dims.
 //   * Everything is computed transposed: Sᵀ = K·Qᵀ (A = K rows from LDS,
 //     B = the wave's Q rows held in registers for the whole kernel) and
 //     Oᵀ += Vᵀ·Pᵀ. In the MFMA output layout lane (r, f), r = lane % 32,
@@ -88,7 +91,8 @@ __device__ __forceinline__ s4 read_tr(const char* at) {
 
 // The gate's σ: the hardware exp, and 1 / d from the hardware reciprocal (one ulp off at worst) and a Newton step, which
 // makes it the full division's value. For the 64 outputs of a lane the step takes 0.3 µs at 16 rows, 2 at a single one
-// and none that shows from 32 on; the division took 1.7 at 16 and 1.6 at 2,307 rows. Past 2^100 d is held there (the step is inf · 0 at infinity; σ is 0 in fp16 by far).
+// and none that shows from 32 on; the division took 1.7 at 16 and 1.6 at 2,307 rows. Past 2^100 d is held there (at
+// infinity the step is inf · 0; σ is 0 in fp16 by far).
 __device__ __forceinline__ float sigmoid(float x) {
   const float d = __builtin_elementwise_minimum(1.0f + __expf(-x), 0x1p100f);  // NaN stays NaN
   const float r = __builtin_amdgcn_rcpf(d);

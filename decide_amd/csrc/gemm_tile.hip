@@ -1285,11 +1285,11 @@ static const VariantEntry kVariants[] = {
     // 8 waves, two per SIMD: 256 x 256 and 256 x 224, the wide M = 2307 projections in under three rounds
     {{8, 8, 2, 2, 2}, gemm_tile8_kernel<8, 4, 4>},
     {{8, 7, 2, 2, 2}, gemm_tile8_kernel<8, 4, 3>},
-    // Small tiles with 5-deep rings for 17 to 600 rows. A CU takes in operands at 50-57 GB/s while W streams from
-    // HBM, whatever the ring depth, so below one round of tiles the time goes with the bytes per tile: tiles just
-    // large enough that all the columns fit one round of 256, without split-K where they do (a reduction launch
-    // costs 4-5 us). gate|up: 32 rows 33.4 -> 21.5 us (32 x 96), 64 rows 34.9 -> 24.9 (64 x 96); down: 64 rows
-    // 23.2 -> 17.1 (64 x 96, split 8); qkv|z|b|a: 163 rows 32 -> 28.3 (64 x 160); out: 276 rows 21.6 -> 20.0 (96 x 96).
+    // Small tiles with 5-deep rings (160 x 96: 4-deep) for 1 to 600 rows. A CU takes in operands at 50-57 GB/s while W
+    // streams from HBM, so below one round of tiles the time goes with the bytes per tile: tiles just large enough that
+    // all the columns fit one round of 256, without split-K where they do (a reduction launch costs 4-5 us). gate|up:
+    // 32 rows 33.4 -> 21.5 us (32 x 96), 64 rows 34.9 -> 24.9 (64 x 96); down: 64 rows 23.2 -> 17.1 (64 x 96, split 8);
+    // qkv|z|b|a: 163 rows 32 -> 28.3 (64 x 160); out: 276 rows 21.6 -> 20.0 (96 x 96).
     {{2, 3, 2, 2}, gemm_tile22_kernel<2, 3, 5, 5, true>},
     {{2, 5, 2, 2}, gemm_tile22_kernel<2, 5, 5, 5, true>},
     {{3, 3, 2, 2}, gemm_tile22_kernel<3, 3, 5, 5, true>},
