@@ -90,8 +90,8 @@ __device__ __forceinline__ s4 read_tr(const char* at) {
 }
 
 // The gate's σ: the hardware exp, and 1 / d from the hardware reciprocal (one ulp off at worst) and a Newton step, which
-// makes it the full division's value. For the 64 outputs of a lane the step takes 0.3 µs at 16 rows, 2 at a single one
-// and none that shows from 32 on; the division took 1.7 at 16 and 1.6 at 2,307 rows. Past 2^100 d is held there (at
+// makes it the full division's value. For the 64 outputs of a lane the step takes 0.3 µs at 16 rows and none that shows
+// from 32 on; the division took 1.7 at 16 and 1.6 at 2,307 rows. Past 2^100 d is held there (at
 // infinity the step is inf · 0; σ is 0 in fp16 by far).
 __device__ __forceinline__ float sigmoid(float x) {
   const float d = __builtin_elementwise_minimum(1.0f + __expf(-x), 0x1p100f);  // NaN stays NaN
@@ -308,17 +308,29 @@ __global__ __launch_bounds__(512) void attention_kernel(const _Float16* __restri
     const int e = 4 * (i % 4);
     xo[(wave * 16 + i) * 64 + lane] = f4{o[e], o[e + 1], o[e + 2], o[e + 3]};
   }
+  // For up to four rows σ is formed here, where the wave would wait for its partner, for more it overlaps the exchange's
+  // reads below. Here and below: 1 row 9.4 and 13.0 µs, 3 rows at position 600 22.6 and 26.3, 6 and 8 rows alike, 32 rows
+  // 13.0 and 11.8.
+  const bool few = rows - qb * kBQ <= 4;
+  if (whole && few) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) gate[i][e] = sigmoid(gate[i][e]);
+  }
   __syncthreads();
   if (qb * kBQ + r >= rows) return;
   const f2 pml = xml[partner * 64 + lane];
   const float mx = fmaxf(m, pml[0]);
   const float wme = exp2f(m - mx), wpa = exp2f(pml[0] - mx);
   const float lt = l * wme + pml[1] * wpa;
-  auto merged = [&](int i) {  // dims 128 half + 8i + 4f .. + 3
+  // dims 128 half + 8i + 4f .. + 3; which product is fused is written out: left to the compiler it differed between the
+  // two uses below, and with it a row's bits by how many rows it is called with
+  auto merged = [&](int i) {
     const f4 po = xo[(partner * 16 + i) * 64 + lane];
     f4 o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = oacc[i / 4][4 * (i % 4) + e] * wme + po[e] * wpa;
+    for (int e = 0; e < 4; ++e) o[e] = fmaf(po[e], wpa, oacc[i / 4][4 * (i % 4) + e] * wme);
     return o;
   };
   if (!whole) {
@@ -338,15 +350,21 @@ __global__ __launch_bounds__(512) void attention_kernel(const _Float16* __restri
   }
   const float inv = 1.0f / lt;
   _Float16* yp = y + (size_t)row * kQDim + h * kHD + 128 * half + 4 * f;
+  auto store = [&](auto sigma) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const f4 o = merged(i);
-    _Float16 v[4];
+    for (int i = 0; i < 16; ++i) {
+      const f4 o = merged(i);
+      _Float16 v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (_Float16)(o[e] * inv * sigmoid(gate[i][e]));
-    *(h2*)(yp + 8 * i) = h2{v[0], v[1]};  // 4-byte alignment suffices (decide's contract)
-    *(h2*)(yp + 8 * i + 2) = h2{v[2], v[3]};
-  }
+      for (int e = 0; e < 4; ++e) v[e] = (_Float16)(o[e] * inv * sigma(gate[i][e]));
+      *(h2*)(yp + 8 * i) = h2{v[0], v[1]};  // 4-byte alignment suffices (decide's contract)
+      *(h2*)(yp + 8 * i + 2) = h2{v[2], v[3]};
+    }
+  };
+  if (few)
+    store([](float x) { return x; });
+  else
+    store([](float x) { return sigmoid(x); });
 }
 
 // Merges the pieces of every query block that has more than one: a workgroup

@@ -443,13 +443,13 @@ def test_attention_key_pieces_keep_rows_independent(gpu, kernels, stream):
                                        err_msg=f"row {r} at {qpos[r]}")
 
 
-@pytest.mark.parametrize("rows", [1, 96])
+@pytest.mark.parametrize("rows", [1, 4, 5, 96])
 def test_attention_gate_is_divided_exactly(gpu, kernels, stream, rows):
     """Row 0 sees one key whose values are 1, so its outputs are the gates' σ = 1 / d in fp16, from the attention kernel
-    (1 row) and from the one that merges key pieces (96 rows). The gates give d = 1 + e^-x an exact fp32 value, chosen so
-    that 1 / d rounds to within an ulp of a tie between two fp16 values: one ulp off in the division shows.
-    e < 0.087 keeps the errors of e (three roundings of at most 2^-22 each) below half an ulp of d. Infinite gates
-    give 1, 0 and NaN as they should."""
+    (on both sides of 4 rows, up to which it forms them earlier) and from the one that merges key pieces (96 rows). The
+    gates give d = 1 + e^-x an exact fp32 value, chosen so that 1 / d rounds to within an ulp of a tie between two fp16
+    values: one ulp off in the division shows. e < 0.087 keeps the errors of e (three roundings of at most 2^-22 each)
+    below half an ulp of d. Infinite gates give 1, 0 and NaN as they should."""
     ties = (2 * np.arange(1024) + 1) / 4096 + 0.5
     d = np.float32(1 / ties[ties > 0.92])[:, None] + np.float32(2.0**-23) * np.arange(-2, 3, dtype=np.float32)
     d = d[d < np.float32(1.087)]
@@ -463,7 +463,7 @@ def test_attention_gate_is_divided_exactly(gpu, kernels, stream, rows):
     want = np.full(4096, 0.5, np.float16)
     want[:len(d)] = sigma.astype(np.float16)
     want[-4:] = [1, 0, np.nan, 0]
-    q, kc, vc, pq, qpos = _attention_case(rows, 1001, [0] + [1000] * (rows - 1), 240)
+    q, kc, vc, pq, qpos = _attention_case(rows, 1001, [0] + [1000 if rows == 96 else 20] * (rows - 1), 240)
     vc[0] = 1
     pq[0, 4096:8192] = gate
     y = empty((rows, 4096), np.float16)
