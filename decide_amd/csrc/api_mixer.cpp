@@ -97,10 +97,10 @@ int dh_gated_delta(dh_ctx* ctx, void* stream, const float* q, const float* k, co
   if (!ctx) return fail(DH_EINVAL, "delta: null context");
   const bool chunked = (ctx->flags & DH_DELTA_CHUNKED) ||
                        (!(ctx->flags & DH_DELTA_SEQUENTIAL) && t >= DH_DELTA_CHUNK_MIN_T);
-  // Between the two: blocks of 16 tokens. The block kernel's start takes as long as 24 tokens one by one, and its time
-  // rises by whole blocks: 17 tokens 8.8 us against 6.8 token by token, 32 9.0 against 9.3, 33 10.1 against 9.4, 36 10.2
-  // against 10.0, 37 10.1 against 10.2, 41 10.1 against 10.9, 169 22.1 against 31.5, 319 35.5 against 55.4. From 320 on
-  // the chunked kernels, which take the conv step in: at 319 tokens conv and recurrence together 47 us either way.
+  // Between the two: blocks of 16 tokens. Two blocks take as long as 30 tokens one by one, and the time rises by whole
+  // blocks: 17 tokens 8.8 us against 6.8 token by token, 32 9.0 against 9.3, 33 10.1 against 9.4, 36 10.2 against 10.0,
+  // 37 10.1 against 10.2, 41 10.1 against 10.9, 169 22.1 against 31.5, 319 35.5 against 55.4. From 320 on the chunked
+  // kernels, which take the conv step in: at 319 tokens conv and recurrence together 47 us either way.
   if (!chunked && !(ctx->flags & DH_DELTA_SEQUENTIAL) && t > kDeltaTokenMaxT) {
     mark(ctx, kKidDeltaBlock);
     return hip_status(dh::launch_gated_delta_block(q, k, v, a, b, a_log, dt_bias, state_in, state_out, o, t, ldab,

@@ -131,7 +131,7 @@ def full_depth_drift(kernels):
 
 @pytest.mark.xfail(strict=False, reason="a max of 22 logits is 0.006 to 0.018 at this depth, whatever the order of the "
                                         "sums: over eight seeds 0.0064-0.0124 for the fp32-sum oracle itself, "
-                                        "0.0067-0.0127 for the token-by-token recurrence, 0.0069-0.0151 for this build")
+                                        "0.0067-0.0127 with the token-by-token recurrence, 0.0069-0.0151 with the block kernel")
 def test_forward_at_full_depth_is_within_the_fp32_noise_floor(gpu, full_depth_drift):
     (diff, _), (floor, _) = full_depth_drift
     assert floor > 0.0
@@ -141,8 +141,8 @@ def test_forward_at_full_depth_is_within_the_fp32_noise_floor(gpu, full_depth_dr
 def test_forward_at_full_depth_is_as_close_as_the_fp32_sum_oracle(gpu, full_depth_drift):
     """The distance of the fp32-sum oracle from the f64 one is the noise floor: a last bit of an fp32 sum flips an fp16
     rounding, and 36 layers amplify it. Over eight seeds that oracle's rms distance is 0.0031 to 0.0045, and that of
-    eight builds of the kernels, whose sums run in other orders, 0.0031 to 0.0059, with no build better than another on
-    average (0.0042 to 0.0045). Held to twice the floor's: over those seeds and builds the ratio is 0.8 to 1.8 (two rms
+    nine versions of the kernels, whose sums run in other orders, 0.0031 to 0.0059, with none better than another on
+    average (0.0042 to 0.0045). Held to twice the floor's: over those seeds and versions the ratio is 0.8 to 1.8 (two rms
     of about ten independent values each: three answer rows), at this seed 0.9 to 1.2."""
     (diff, rms), (_, floor) = full_depth_drift
     assert 0.0 < floor
